@@ -1,6 +1,7 @@
 """Compile the HIP library in-tree for gfx950: publicrelease_2020_amd/libflosic_hip.so."""
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import subprocess
 import sys
@@ -9,15 +10,21 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libflosic_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-SOURCES = ["flosic_kernels.hip", "flosic_api.hip"]
+SOURCES = ["flosic_kernels.hip", "flosic_coulomb_fp.hip", "flosic_coulomb_bf16.hip", "flosic_api.hip"]
+HIPCC = os.path.join(ROCM, "bin", "hipcc")
+OBJ = os.path.join(HERE, "_build")
 
 
-def command(out: str = LIB) -> list:
-    return [os.path.join(ROCM, "bin", "hipcc"), "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+def compile_command(src: str, obj: str) -> list:
+    return [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
             # packed FP32 instructions are kept out of all device code
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
             "-Wno-unused-command-line-argument",
-            "-I" + os.path.join(ROCM, "include"), *[os.path.join(CSRC, s) for s in SOURCES],
+            "-I" + os.path.join(ROCM, "include"), "-c", os.path.join(CSRC, src), "-o", obj]
+
+
+def link_command(objs: list, out: str) -> list:
+    return [HIPCC, "--offload-arch=gfx950", "-fPIC", "-shared", *objs,
             "-L" + os.path.join(ROCM, "lib"), "-lrocblas", "-Wl,-rpath," + os.path.join(ROCM, "lib"), "-o", out]
 
 
@@ -49,15 +56,25 @@ def build_fortran(verbose: bool = False) -> str:
     return FORTRAN_EXE
 
 
-def build(verbose: bool = False) -> str:
-    tmp = LIB + ".tmp"
-    cmd = command(tmp)
+def _run(cmd: list, verbose: bool, what: str) -> None:
     if verbose:
         print(" ".join(cmd))
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed building libflosic_hip.so")
+        raise RuntimeError("hipcc failed " + what)
+
+
+def build(verbose: bool = False) -> str:
+    """Every source in a compiler process of its own, at once; then the link."""
+    os.makedirs(OBJ, exist_ok=True)
+    objs = [os.path.join(OBJ, os.path.splitext(s)[0] + ".o") for s in SOURCES]
+    with concurrent.futures.ThreadPoolExecutor(len(SOURCES)) as pool:
+        jobs = [pool.submit(_run, compile_command(s, o), verbose, "compiling " + s) for s, o in zip(SOURCES, objs)]
+        for j in jobs:
+            j.result()
+    tmp = LIB + ".tmp"
+    _run(link_command(objs, tmp), verbose, "linking libflosic_hip.so")
     os.replace(tmp, LIB)
     return LIB
 
