@@ -160,13 +160,13 @@ struct flosic_ctx {
     std::vector<int32_t> pair_list;  // 6 per shell pair, canonical order
     int npair = 0;                   // screened primitive shell pairs
     int ngroup = 0, nrows = 0;       // exponent-pair groups and their Hermite rows
-    int segL[6] = {0, 0, 0, 0, 0, 0};
+    FpSegs segL = {{0, 0, 0, 0, 0, 0}};  // the groups by order
     DevBuf<int> d_ps_f0, d_ps_stride, d_ps_ncart, d_ps_c0, d_ps_nc, d_pair_row;
     DevBuf<double> d_ps_coef;
     DevBuf<PairDev> d_pairs;
-    DevBuf<ChunkDev> d_chunks, d_chunks_bf16;
-    int nchunks = 0, nchunks_bf16 = 0;
-    int64_t rows_padded = 0, rows_padded_bf16 = 0;
+    DevBuf<ChunkDev> d_chunks_bf16;
+    int nchunks_bf16 = 0;
+    int64_t rows_padded = 0, rows_padded_bf16 = 0;  // Hermite rows as the FP and the split-BF16 kernels stream them
     DevBuf<double> d_lapplane, d_lap, d_pot, d_wop, d_small, d_B, d_hao;  // LAGMULT_SLV / AO SIC Hamiltonian
     DevBuf<double> d_scf;  // SCFSICW orbital update: ham_ao, ham_ao C, C^T ham_ao C
     bool lapplane_ok = false;
@@ -202,7 +202,8 @@ struct flosic_ctx {
     // spins
     Spin sp[2];
     // evaluation buffers
-    int nF = 0, ldh = 0;
+    int nF = 0, ldh = 0;  // ldh: nF rounded up to the widest column block (the legal block widths divide it)
+    int ldc = 0;          // leading dimension of H: nF rounded up to 16, ldh for the split-BF16 forms
     DevBuf<double> d_fodxyz, d_fodchi;  // FOD coordinates of both spins (x, y, z arrays), basis planes at them
     DevBuf<double> d_cflo, d_dps, d_H, d_phi, d_VH, d_Vtot, d_U, d_part, d_energy, d_G, d_Gpart, d_vabpart, d_vab,
         d_lambda, d_asy, d_Ux, d_lamex, d_dft, d_dftpart, d_dplanes, d_dphi, d_dvt, d_du, d_dG;
@@ -789,11 +790,10 @@ int build_pairs(flosic_ctx *c) {
                              (p.a * p.A[2] + p.b * p.B[2]) / pe, pe);
     }
     c->nrows = row;
-    // chunk lists: consecutive groups of one L, at most `cap_rows` rows, zero-extended to a multiple of `quant`.  With
-    // split_l4 (the split-BF16 list, 32-row steps) the L = 4 groups (35 rows) go into two chunk types instead: chunk
-    // type 5 holds the first 32 rows of two groups, type 6 the last 3 rows of 21 groups; a whole 35-row group would
-    // pad its 64-row chunk with 29 zero rows.
-    auto make_chunks = [&](int cap_rows, int quant, int64_t &padded, bool split_l4) {
+    // split-BF16 chunk list: consecutive groups of one L, at most `cap_rows` rows, zero-extended to a multiple of `quant`.
+    // The L = 4 groups (35 rows) go into two chunk types instead: chunk type 5 holds the first 32 rows of two groups,
+    // type 6 the last 3 rows of 21 groups; a whole 35-row group would pad its 64-row chunk with 29 zero rows.
+    auto make_chunks = [&](int cap_rows, int quant, int64_t &padded) {
         std::vector<ChunkDev> out;
         padded = 0;
         auto emit = [&](int k, int e, int type, int rpg) {
@@ -804,7 +804,7 @@ int build_pairs(flosic_ctx *c) {
         for (int k = 0; k < c->ngroup;) {
             const int L = pairs[k].lA + pairs[k].lB;
             const int nt = (L + 1) * (L + 2) * (L + 3) / 6;
-            if (split_l4 && L == 4) {
+            if (L == 4) {
                 int end = k;
                 while (end < c->ngroup && pairs[end].lA + pairs[end].lB == 4) ++end;
                 for (int type = 5; type <= 6; ++type) {
@@ -822,19 +822,18 @@ int build_pairs(flosic_ctx *c) {
         }
         return out;
     };
-    const std::vector<ChunkDev> chunks = make_chunks(kChunkRows, 4, c->rows_padded, false);
-    const std::vector<ChunkDev> chunks16 = make_chunks(kChunkRowsBf16, 32, c->rows_padded_bf16, true);
-    c->nchunks = (int)chunks.size();
+    const std::vector<ChunkDev> chunks16 = make_chunks(kChunkRowsBf16, 32, c->rows_padded_bf16);
     c->nchunks_bf16 = (int)chunks16.size();
     // segment offsets: segL[L] = first group with lA+lB >= L
     for (int L = 0; L <= 5; ++L) {
         int k = 0;
         while (k < c->ngroup && pairs[k].lA + pairs[k].lB < L) ++k;
-        c->segL[L] = k;
+        c->segL.g[L] = k;
     }
+    c->rows_padded = 4 * fp_steps(c->segL);
     int r = 0;
     if ((r = upload(c, c->d_pairs, pairs)) || (r = upload(c, c->d_pairP, pP)) || (r = upload(c, c->d_pair_row, prow)) ||
-        (r = upload(c, c->d_chunks, chunks)) || (r = upload(c, c->d_chunks_bf16, chunks16)) ||
+        (r = upload(c, c->d_chunks_bf16, chunks16)) ||
         (r = upload(c, c->d_ps_f0, ps_f0)) || (r = upload(c, c->d_ps_stride, ps_stride)) ||
         (r = upload(c, c->d_ps_ncart, ps_ncart)) || (r = upload(c, c->d_ps_c0, ps_c0)) ||
         (r = upload(c, c->d_ps_nc, ps_nc)) || (r = upload(c, c->d_ps_coef, ps_coef)))
@@ -1040,7 +1039,7 @@ void coulomb_launch(flosic_ctx *c, const double *x, const double *y, const doubl
     const int nF = c->nF;
     switch (coulomb_form(c)) {
         case COUL_VALU:
-            launch_coulomb(c->segL, c->d_pairP.p, c->d_pair_row.p, c->d_H.p, c->ldh, x, y, z, M, c->d_btab.p, nF, V,
+            launch_coulomb(c->segL.g, c->d_pairP.p, c->d_pair_row.p, c->d_H.p, c->ldc, x, y, z, M, c->d_btab.p, nF, V,
                            ldv, c->stream);
             break;
         case COUL_BF16: {
@@ -1052,12 +1051,12 @@ void coulomb_launch(flosic_ctx *c, const double *x, const double *y, const doubl
             break;
         }
         case COUL_FP32:
-            launch_coulomb_mfma<float>(c->d_chunks.p, c->nchunks, c->rows_padded / 4, c->d_pairP.p, c->d_H32.p, c->ldh,
-                                       x, y, z, M, c->d_btab.p, nF, V, ldv, c->stream, nfb);
+            launch_coulomb_mfma<float>(c->segL, c->d_pairP.p, c->d_H32.p, x, y, z, M, c->d_btab.p, nF, V, ldv, c->stream,
+                                       nfb);
             break;
         case COUL_FP64:
-            launch_coulomb_mfma<double>(c->d_chunks.p, c->nchunks, c->rows_padded / 4, c->d_pairP.p, c->d_H64.p,
-                                        c->ldh, x, y, z, M, c->d_btab.p, nF, V, ldv, c->stream, nfb);
+            launch_coulomb_mfma<double>(c->segL, c->d_pairP.p, c->d_H64.p, x, y, z, M, c->d_btab.p, nF, V, ldv, c->stream,
+                                        nfb);
             break;
     }
 }
@@ -1149,6 +1148,7 @@ int eval_fo(flosic_ctx *c) {
     {
         const int nfb = coulomb_cols(nF);
         c->ldh = (nF + nfb - 1) / nfb * nfb;
+        c->ldc = coulomb_form(c) == COUL_BF16 ? c->ldh : (nF + 15) / 16 * 16;
     }
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipEventRecord(c->ev[EV_START], c->stream));
@@ -1196,8 +1196,8 @@ int eval_hermite(flosic_ctx *c) {
     ALLOC(c, c->d_dps, (size_t)nps * 6 * nF);
     launch_prim_coef(nps, c->d_ps_f0.p, c->d_ps_stride.p, c->d_ps_ncart.p, c->d_ps_c0.p, c->d_ps_nc.p, c->d_ps_coef.p,
                      c->d_cflo.p, nF, N, c->d_dps.p, c->stream);
-    ALLOC(c, c->d_H, (size_t)c->nrows * c->ldh);
-    launch_hermite(c->ngroup, c->d_pairs.p, c->d_dps.p, nF, c->d_H.p, c->ldh, c->stream);
+    ALLOC(c, c->d_H, (size_t)c->nrows * c->ldc);
+    launch_hermite(c->ngroup, c->d_pairs.p, c->d_dps.p, nF, c->d_H.p, c->ldc, c->stream);
     HIPCHK(c, hipGetLastError());
     MARK(c, EV_HERM);
     // the Coulomb operand in MFMA order
@@ -1214,12 +1214,12 @@ int eval_hermite(flosic_ctx *c) {
             break;
         }
         case COUL_FP32:
-            ALLOC(c, c->d_H32, (size_t)c->rows_padded * c->ldh);
-            launch_frag_h<float>(c->d_chunks.p, c->nchunks, c->d_H.p, c->ldh, nF, c->d_H32.p, c->stream);
+            ALLOC(c, c->d_H32, (size_t)c->rows_padded * c->ldc);
+            launch_frag_h<float>(c->segL, c->d_H.p, c->ldc, nF, c->d_H32.p, c->stream);
             break;
         case COUL_FP64:
-            ALLOC(c, c->d_H64, (size_t)c->rows_padded * c->ldh);
-            launch_frag_h<double>(c->d_chunks.p, c->nchunks, c->d_H.p, c->ldh, nF, c->d_H64.p, c->stream);
+            ALLOC(c, c->d_H64, (size_t)c->rows_padded * c->ldc);
+            launch_frag_h<double>(c->segL, c->d_H.p, c->ldc, nF, c->d_H64.p, c->stream);
             break;
         default: break;
     }
@@ -1518,12 +1518,13 @@ CoulJob<double> coulomb_job(const flosic_ctx *c) {
     CoulJob<double> J{};
     const CoulForm form = coulomb_form(c);
     const int nfb = coulomb_nfb(c);
-    J.chunks = form == COUL_BF16 ? c->d_chunks_bf16.p : c->d_chunks.p;
-    J.nchunks = form == COUL_BF16 ? c->nchunks_bf16 : c->nchunks;
+    J.chunks = c->d_chunks_bf16.p;
+    J.nchunks = c->nchunks_bf16;
+    J.seg = c->segL;
     J.pP = c->d_pairP.p;
     J.H = form == COUL_BF16 ? (const void *)c->d_Hs.p : form == COUL_FP32 ? (const void *)c->d_H32.p
                                                                            : (const void *)c->d_H64.p;
-    J.nct = c->ldh / 16;
+    J.nct = c->ldc / 16;
     J.X = c->d_x.p;
     J.Y = c->d_y.p;
     J.Z = c->d_z.p;
@@ -1532,7 +1533,7 @@ CoulJob<double> coulomb_job(const flosic_ctx *c) {
     J.V = c->d_VH.p;
     J.ldv = c->M;
     J.nsteps = form == COUL_BF16 ? c->rows_padded_bf16 / 32 : c->rows_padded / 4;
-    J.ncb = c->ldh / nfb;
+    J.ncb = form == COUL_BF16 ? c->ldh / nfb : fp_col_blocks(c->nF, nfb);
     J.nfb = nfb;
     const bool far = form == COUL_BF16 && c->prec == FLOSIC_PREC_BF16X3 && c->far_ok && c->far_words > 0;
     J.far = far ? c->d_far.p : nullptr;
@@ -1550,7 +1551,7 @@ int build_plan(flosic_batch *b) {
     for (int i = 0; i < (int)b->ctxs.size(); ++i) {
         const flosic_ctx *c = b->ctxs[i];
         const CoulForm form = coulomb_form(c);
-        if (form == COUL_VALU || c->nchunks <= 0) continue;
+        if (form == COUL_VALU || c->ngroup <= 0) continue;
         const int np = form == COUL_BF16 ? (c->prec == FLOSIC_PREC_BF16X3 ? 3 : 2) : 0;
         auto it = std::find_if(b->classes.begin(), b->classes.end(), [&](const flosic_batch::Class &k) {
             return k.form == form && k.npieces == np;

@@ -30,9 +30,6 @@ __device__ __forceinline__ void advance(SubStep &p, const ChunkDev *chunks, int 
 // LAYOUT 2: Rl[point * LD + row] in T.  Share 0 also zeroes the rows beyond the groups.
 // R is computed in FP64 for the FP64 form and in FP32 for the FP32 and split-BF16 operands, with the Boys table of
 // that precision (the FP32 copy follows the FP64 table in device memory; the split-BF16 kernel reads it from LDS)
-template <typename T>
-using RType = typename std::conditional<sizeof(T) == 8, double, float>::type;
-
 // RPG rows per group from Hermite row ROFF on (the whole group by default; the split-BF16 list's L = 4 head / tail
 // chunks take rows [0, 32) / [32, 35) of each group, see chunk_rpg)
 template <int L, typename T, int LD, int LAYOUT, int NP, int RPG = ntuv(L), int ROFF = 0>
@@ -490,7 +487,7 @@ void launch_coulomb_bf16(int npieces, const ChunkDev *chunks, int nchunks, int64
     if (nchunks <= 0 || M <= 0) return;
     if (nfb <= 0) nfb = coulomb_cols_split(nF);
     const CoulJob<__bf16> J{chunks, nchunks, pairP, Hs, ldh / 16, x, y, z, M, nF, V, ldv, nsteps, ldh / nfb, nfb,
-                            npieces == 3 ? far : nullptr, npieces == 3 ? farw : 0};
+                            npieces == 3 ? far : nullptr, npieces == 3 ? farw : 0, FpSegs{}};
     const dim3 grid((unsigned)((M + 63) / 64), (unsigned)(ldh / nfb)), blk(kCoulThreads);
 #define FLOSIC_WSB(NP, NFB) hipLaunchKernelGGL((k_coulomb_ws_bf16<NP, NFB>), grid, blk, 0, s, J, btab)
 #define FLOSIC_WSB_NFB(NP)                        \

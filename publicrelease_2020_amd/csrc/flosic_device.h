@@ -188,6 +188,10 @@ __device__ __forceinline__ ChunkDev chunk_at(const ChunkDev *__restrict__ chunks
     __builtin_memcpy(&ch, w, sizeof(ch));
     return ch;
 }
+// the type in which R is generated: FP64 for the FP64 form, FP32 for the FP32 and split-BF16 operands
+template <typename T>
+using RType = typename std::conditional<sizeof(T) == 8, double, float>::type;
+
 template <typename T> struct MfmaTraits;
 // Operands of both 16x16x4 forms: lane l holds A[l%16][l/16] and B[l/16][l%16].  The accumulators differ:
 // FP32 register r of lane l holds D[4*(l/16) + r][l%16], FP64 register r holds D[l/16 + 4*r][l%16].

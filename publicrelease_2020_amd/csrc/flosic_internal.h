@@ -40,28 +40,32 @@ struct PairDev {
     double sym;          // 2 for cA != cB, else 1
 };
 
-// chunk of consecutive groups of one order L: Hermite rows [hrow0, hrow0 + (pe-pb)*ntuv(L)) staged in LDS and
-// zero-extended to kr rows (a multiple of the MFMA K step of the kernel that uses the chunk list)
-constexpr int kChunkRows = 64;      // FP64 / FP32 MFMA kernels: K step 4
+// chunk of consecutive groups of one order L (split-BF16 forms): Hermite rows [hrow0, hrow0 + (pe-pb)*ntuv(L)) staged
+// in LDS and zero-extended to kr rows (a multiple of the MFMA K step)
 constexpr int kChunkRowsBf16 = 64;  // split-BF16 kernel: K step 32
 constexpr int kFarWords = 1000;     // far-chunk bits per tile the split-BF16 kernel holds in LDS (32000 chunks)
 struct ChunkDev {
-    // groups [pb, pe); L: their Hermite order, or in the split-BF16 list 5 / 6 for the first 32 / last 3 rows of
-    // L = 4 groups; kr: rows after zero extension; hrow0: first Hermite row of group pb
+    // groups [pb, pe); L: their Hermite order, or 5 / 6 for the first 32 / last 3 rows of L = 4 groups; kr: rows after zero extension; hrow0: first Hermite row of group pb
     int pb, pe, L, kr, hrow0;
     int prow0;  // first row of the chunk in the zero-extended row space of its list (split-BF16 H layout)
 };
 
+// the groups by order: those of order L are [g[L], g[L + 1])
+struct FpSegs {
+    int g[6];
+};
+
 // One system's Coulomb contraction as the kernels see it.  H is in the operand order of the form (double or
 // float fragments over K steps of 4 rows, or bf16 pieces over K steps of 32 rows: nsteps steps); ncb column
-// blocks of NFB columns; V[f * ldv + k].
+// blocks (split-BF16: of nfb columns; FP forms: the nct column tiles shared out evenly); V[f * ldv + k].  The FP forms
+// walk the groups by seg, the split-BF16 forms by the chunk list.
 template <typename T>
 struct CoulJob {
     const ChunkDev *chunks;
     int nchunks;
     const double4 *pP;
     const void *H;
-    int nct;  // ldh / 16
+    int nct;  // 16-column tiles of H
     const double *X, *Y, *Z;
     int64_t M;
     int nF;
@@ -73,13 +77,14 @@ struct CoulJob {
     // three-piece split-BF16 form: far-chunk bits of every 64-point tile (farw words per tile), or null
     const unsigned *far;
     int farw;
+    FpSegs seg;
 };
 
-// Column-block widths the Coulomb kernels are built for: nfb must divide ldh; the split-BF16 form takes at most 192
+// Column-block widths that may be asked for: nfb must divide ldh (nF rounded up to a multiple of coulomb_cols); the
+// split-BF16 form takes at most 192
 bool coulomb_cols_legal(int nfb, int ldh, bool split);
 
-// FLO columns handled by one Coulomb block: all of them up to 256; the H leading dimension ldh is nF rounded
-// up to a multiple of this
+// FLO columns handled by one Coulomb block: all of them up to 256
 int coulomb_cols(int nF);
 
 // per-phase launch helpers (stream-ordered)
@@ -110,16 +115,17 @@ void launch_coulomb(const int *segL /*6 offsets*/, const double4 *pairP, const i
                     int ldh, const double *x, const double *y, const double *z, int64_t M, const double *btab,
                     int nF, double *V, int64_t ldv, hipStream_t s);
 
-// MFMA forms.  H is first rearranged into MFMA operand order over the chunk list's zero-extended rows
-// (nsteps K steps: rows/4 for the FP64/FP32 list, rows/32 for the bf16 list); the Coulomb kernels then generate
-// R_tuv of every (point, group) once and stream H.  T = double (FP64 MFMA) or float (FP32 MFMA, FP64 sums per
-// chunk).
+// MFMA forms.  H (leading dimension ldh, a multiple of 16) is first rearranged into MFMA operand order; the Coulomb
+// kernels then generate R_tuv of every (point, group) and stream H.  T = double (FP64 MFMA) or float (FP32 MFMA, FP64
+// sums per chunk of <= 64 rows): fp_steps K steps of 4 rows, at most nfb FLO columns per block.
+int64_t fp_steps(const FpSegs &seg);
+int fp_col_blocks(int nF, int nfb);
 template <typename T>
-void launch_frag_h(const ChunkDev *chunks, int nchunks, const double *H, int ldh, int nF, T *Hf, hipStream_t s);
+void launch_frag_h(const FpSegs &seg, const double *H, int ldh, int nF, T *Hf, hipStream_t s);
 template <typename T>
-void launch_coulomb_mfma(const ChunkDev *chunks, int nchunks, int64_t nsteps, const double4 *pairP, const T *Hf,
-                         int ldh, const double *x, const double *y, const double *z, int64_t M, const double *btab,
-                         int nF, double *V, int64_t ldv, hipStream_t s, int nfb = 0);
+void launch_coulomb_mfma(const FpSegs &seg, const double4 *pairP, const T *Hf, const double *x, const double *y,
+                         const double *z, int64_t M, const double *btab, int nF, double *V, int64_t ldv, hipStream_t s,
+                         int nfb = 0);
 
 // Batched form: every job of one Coulomb form in one launch over the (system, point tile, column block) items; the
 // job records and the item offsets in device memory (off[j] the first item of job j, which has ceil(M/64) * ncb items,
