@@ -10,7 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libflosic_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-SOURCES = ["flosic_kernels.hip", "flosic_coulomb_fp64.hip", "flosic_coulomb_fp32.hip", "flosic_coulomb_bf16.hip", "flosic_api.hip"]
+SOURCES = ["flosic_kernels.hip", "flosic_gemm.hip", "flosic_coulomb_fp64.hip", "flosic_coulomb_fp32.hip", "flosic_coulomb_bf16.hip", "flosic_api.hip"]
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 OBJ = os.path.join(HERE, "_build")
 

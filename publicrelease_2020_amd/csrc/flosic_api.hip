@@ -967,28 +967,37 @@ int run_frmorb(flosic_ctx *c) {
     return 0;
 }
 
-// out (rows x n, column-major) (+)= A^T B with A (M x rows) and B (M x n) column-major, leading dimension M: the
-// point dimension is split into slices (the products are skinny with K = M) and the slice partials are summed
-// in a fixed order, onto out when accumulate is set
+// out (rows x n, column-major) (+)= sum over nplane planes of A^T B, A (M x rows) and B (M x n) column-major with leading
+// dimensions lda, ldb (default M) and plane strides sa, sb: the points are split into slices whose partials are summed in
+// a fixed order, onto out when accumulate is set
 int gemm_tn_points(flosic_ctx *c, int rows, int n, const double *A, const double *B, int64_t M, double *out,
-                   bool accumulate = false, int64_t lda = 0, int64_t ldb = 0) {
+                   bool accumulate = false, int64_t lda = 0, int64_t ldb = 0, int nplane = 1, int64_t sa = 0,
+                   int64_t sb = 0) {
     if (rows <= 0 || n <= 0) return 0;
     if (lda <= 0) lda = M;
     if (ldb <= 0) ldb = M;
-    const double one = 1.0, zero = 0.0;
-    int nsl = 64;
-    while (nsl > 1 && M / nsl < 4096) --nsl;
-    const int64_t ms = M / nsl, rest = M - ms * nsl;  // nsl slices of ms points, then the remainder
-    ALLOC(c, c->d_Gpart, (size_t)(nsl + 1) * rows * n);
-    BLASCHK(c, rocblas_dgemm_strided_batched(c->blas, rocblas_operation_transpose, rocblas_operation_none, rows, n,
-                                             (rocblas_int)ms, &one, A, (rocblas_int)lda, ms, B, (rocblas_int)ldb, ms,
-                                             &zero, c->d_Gpart.p, rows, (rocblas_stride)rows * n, nsl));
-    int nparts = nsl;
-    if (rest > 0) {
-        BLASCHK(c, rocblas_dgemm(c->blas, rocblas_operation_transpose, rocblas_operation_none, rows, n,
-                                 (rocblas_int)rest, &one, A + ms * nsl, (rocblas_int)lda, B + ms * nsl,
-                                 (rocblas_int)ldb, &zero, c->d_Gpart.p + (size_t)nsl * rows * n, rows));
-        nparts = nsl + 1;
+    int nparts;
+    if (rows >= 512 && n > 80 && nplane == 1) {
+        // large in all three dimensions: the library's LDS-tiled product, batched over 64 point slices (1720 x 192 and
+        // 368 437 points: 4.1 ms against 6.0; 916 x 96, 370 513: 1.46 against 1.70; even at 792 x 72, and 128 x 20 with
+        // 69 773 points takes it 0.24 against 0.06, because two dimensions fill too few of its 128 x 64 tiles)
+        const double one = 1.0, zero = 0.0;
+        int nsl = 64;
+        while (nsl > 1 && M / nsl < 4096) --nsl;
+        const int64_t ms = M / nsl, rest = M - ms * nsl;  // nsl slices of ms points, then the remainder
+        nparts = nsl + (rest > 0 ? 1 : 0);
+        ALLOC(c, c->d_Gpart, (size_t)(nsl + 1) * rows * n);
+        BLASCHK(c, rocblas_dgemm_strided_batched(c->blas, rocblas_operation_transpose, rocblas_operation_none, rows, n,
+                                                 (rocblas_int)ms, &one, A, (rocblas_int)lda, ms, B, (rocblas_int)ldb, ms,
+                                                 &zero, c->d_Gpart.p, rows, (rocblas_stride)rows * n, nsl));
+        if (rest > 0)
+            BLASCHK(c, rocblas_dgemm(c->blas, rocblas_operation_transpose, rocblas_operation_none, rows, n,
+                                     (rocblas_int)rest, &one, A + ms * nsl, (rocblas_int)lda, B + ms * nsl,
+                                     (rocblas_int)ldb, &zero, c->d_Gpart.p + (size_t)nsl * rows * n, rows));
+    } else {
+        nparts = tn_slices(rows, n, M, nplane);
+        ALLOC(c, c->d_Gpart, (size_t)nparts * rows * n);
+        launch_tn(A, lda, sa, B, ldb, sb, rows, n, M, nplane, c->d_Gpart.p, c->stream);
     }
     launch_reduce_partials(c->d_Gpart.p, 1, nparts, rows * n, out, c->stream, accumulate);
     HIPCHK(c, hipGetLastError());
@@ -998,12 +1007,8 @@ int gemm_tn_points(flosic_ctx *c, int rows, int n, const double *A, const double
 // phi (nd planes of [ncol][m], plane stride ncol*m) = planes (nd planes of [nbas][m]) . cf (nbas x ncol)
 int orbitals_on_points(flosic_ctx *c, const double *planes, int64_t m, int nd, const double *cf, int ncol,
                        double *phi) {
-    const double one = 1.0, zero = 0.0;
-    const int N = c->nbas;
-    for (int d = 0; d < nd; ++d)
-        BLASCHK(c, rocblas_dgemm(c->blas, rocblas_operation_none, rocblas_operation_none, (rocblas_int)m, ncol, N,
-                                 &one, planes + (size_t)d * N * m, (rocblas_int)m, cf, N, &zero,
-                                 phi + (size_t)d * ncol * m, (rocblas_int)m));
+    launch_orbitals(planes, m, nd, c->nbas, cf, ncol, phi, c->stream);
+    HIPCHK(c, hipGetLastError());
     return 0;
 }
 
@@ -1342,11 +1347,9 @@ int eval_fields(flosic_ctx *c, bool overlap_host = false) {
             for (int s = 0; s < 2; ++s) {
                 const int n = c->sp[s].nocc;
                 const size_t off = s == 0 ? 0 : (size_t)n0;
-                for (int d = 0; d < 4 && n > 0; ++d)
-                    if ((r = gemm_tn_points(c, n, n, c->d_phi.p + ((size_t)d * nF + off) * m,
-                                            c->d_Ux.p + ((size_t)d * nF + off) * m, m, c->d_lamex.p + lo,
-                                            k0 > 0 || d > 0)))
-                        return r;
+                if ((r = gemm_tn_points(c, n, n, c->d_phi.p + off * m, c->d_Ux.p + off * m, m, c->d_lamex.p + lo, k0 > 0,
+                                        0, 0, 4, (int64_t)nF * m, (int64_t)nF * m)))
+                    return r;
                 lo += (size_t)n * n;
             }
         }
@@ -2267,13 +2270,12 @@ int32_t flosic_lagmult_slv(flosic_ctx *c, int32_t ispn, const double *pot, int32
     if (ldsic < n) return fail(c, FLOSIC_EINVAL, "ldsic %d < nfrm %d", ldsic, n);
     if (n == 0) return FLOSIC_OK;
     const int off = s == 0 ? 0 : c->sp[0].nocc;
-    const double one = 1.0, zero = 0.0;
     const double *cf = c->d_cflo.p + (size_t)off * N;
     const bool blocked = c->block_pts > 0;
     const int64_t mb = mesh_block(c);
     const int nd = xc_planes(c);
     if ((r = upload(c, c->d_pot, pot, (size_t)M))) return r;
-    ALLOC(c, c->d_lap, (size_t)n * mb);
+    ALLOC(c, c->d_lap, (size_t)(nd == 10 ? 3 : 1) * n * mb);
     ALLOC(c, c->d_wop, (size_t)n * mb);
     ALLOC(c, c->d_small, (size_t)n * n);
     // Laplacians of the FLOs: from the Hessian planes (PBE) or from a Laplacian plane (kept resident unless in
@@ -2296,18 +2298,15 @@ int32_t flosic_lagmult_slv(flosic_ctx *c, int32_t ispn, const double *pot, int32
             if ((r = orbitals_on_points(c, planes, m, 1, cf, n, c->d_phi.p))) return r;
             phi = c->d_phi.p;
         }
-        if (nd == 10) {
-            for (int d = 4; d < 7; ++d)
-                BLASCHK(c, rocblas_dgemm(c->blas, rocblas_operation_none, rocblas_operation_none, (rocblas_int)m, n, N,
-                                         &one, planes + (size_t)d * N * m, (rocblas_int)m, cf, N,
-                                         d == 4 ? &zero : &one, c->d_lap.p, (rocblas_int)m));
+        if (nd == 10) {  // xx, yy, zz of the FLOs, added up where they are used
+            if ((r = orbitals_on_points(c, planes + (size_t)4 * N * m, m, 3, cf, n, c->d_lap.p))) return r;
         } else {
             if (blocked && (r = block_planes(c, k0, m, -1, c->d_lapplane.p))) return r;
-            BLASCHK(c, rocblas_dgemm(c->blas, rocblas_operation_none, rocblas_operation_none, (rocblas_int)m, n, N, &one,
-                                     c->d_lapplane.p, (rocblas_int)m, cf, N, &zero, c->d_lap.p, (rocblas_int)m));
+            if ((r = orbitals_on_points(c, c->d_lapplane.p, m, 1, cf, n, c->d_lap.p))) return r;
         }
         // T_k = w (-1/2 lap phi_k + V phi_k), L = phi^T T
-        launch_weighted_op(n, m, c->d_w.p + k0, c->d_pot.p + k0, phi, c->d_lap.p, -0.5, c->d_wop.p, c->stream);
+        launch_weighted_op(n, m, c->d_w.p + k0, c->d_pot.p + k0, phi, c->d_lap.p, nd == 10 ? 3 : 1, -0.5,
+                           c->d_wop.p, c->stream);
         HIPCHK(c, hipGetLastError());
         if ((r = gemm_tn_points(c, n, n, phi, c->d_wop.p, m, c->d_small.p, k0 > 0))) return r;
     }
@@ -2343,7 +2342,7 @@ int32_t flosic_sic_hamiltonian(flosic_ctx *c, int32_t ispn, double *hao) {
             if ((r = orbitals_on_points(c, c->d_planes.p, m, 1, c->d_cflo.p + (size_t)off * N, n, c->d_phi.p))) return r;
             phi = c->d_phi.p;
         }
-        launch_weighted_op(n, m, c->d_w.p + k0, nullptr, phi, nullptr, 0.0, c->d_wop.p, c->stream);
+        launch_weighted_op(n, m, c->d_w.p + k0, nullptr, phi, nullptr, 0, 0.0, c->d_wop.p, c->stream);
         HIPCHK(c, hipGetLastError());
         if ((r = gemm_tn_points(c, N, n, c->d_planes.p, c->d_wop.p, m, c->d_B.p, k0 > 0))) return r;
     }

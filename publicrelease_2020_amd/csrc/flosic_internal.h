@@ -98,9 +98,9 @@ template <typename T>
 void launch_basis_planes(const BasisDev &B, const double *x, const double *y, const double *z, int64_t M, int nd,
                          T *phi, int64_t ldphi, hipStream_t s);
 
-// T[f][k] = w_k (a * lap[f][k] + pot[k] * phi[f][k]); lap may be null, pot null means 1
+// T[f][k] = w_k (a * lap[f][k] + pot[k] * phi[f][k]); lap the sum of nlap planes or null, pot null means 1
 void launch_weighted_op(int n, int64_t M, const double *w, const double *pot, const double *phi, const double *lap,
-                        double a, double *T, hipStream_t s);
+                        int nlap, double a, double *T, hipStream_t s);
 
 void launch_prim_coef(int nps, const int *ps_f0, const int *ps_stride, const int *ps_ncart, const int *ps_c0,
                       const int *ps_nc, const double *ps_coef, const double *cflo, int nF, int ldc, double *dps,
@@ -152,6 +152,15 @@ void launch_coulomb_bf16(int npieces, const ChunkDev *chunks, int nchunks, int64
 void launch_far_bits(const double *x, const double *y, const double *z, int64_t M, const ChunkDev *chunks,
                      int nchunks, const double4 *pairP, double tfar, int farw, unsigned *far, double *farrows,
                      hipStream_t s);
+
+// phi[d][f][k] = sum_mu planes[d][mu][k] cf[mu + N f]: nd planes of [N][m] times the N x nc coefficients
+void launch_orbitals(const double *planes, int64_t m, int nd, int N, const double *cf, int nc, double *phi,
+                     hipStream_t s);
+// part[slice][r + rows c], tn_slices(...) slices in all, whose sum is sum_p sum_k A[p sa + k + lda r] B[p sb + k + ldb c]
+// over nplane planes and M points
+int tn_slices(int rows, int n, int64_t M, int nplane);
+void launch_tn(const double *A, int64_t lda, int64_t sa, const double *B, int64_t ldb, int64_t sb, int rows, int n,
+               int64_t M, int nplane, double *part, hipStream_t s);
 
 // XC + total potential + energy partials over M points: phi nd planes of [nF][M] (plane stride nF*M), Vtot and U
 // [nF][M], VH[f * ldvh + k], w[k]; 256-point block b writes partial[(f * nblk + blk0 + b) * 9 + q].  For PBE,

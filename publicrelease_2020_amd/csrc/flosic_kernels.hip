@@ -126,23 +126,27 @@ template void launch_basis_planes<double>(const BasisDev &, const double *, cons
 template void launch_basis_planes<float>(const BasisDev &, const double *, const double *, const double *, int64_t,
                                          int, float *, int64_t, hipStream_t);
 
-// T[f][k] = w_k (a * lap[f][k] + pot[k] * phi[f][k]) over n FLOs (lap may be null: T = w * pot * phi, or with
-// pot null: T = w * phi)
+// T[f][k] = w_k (a * lap[f][k] + pot[k] * phi[f][k]) over n FLOs, lap the sum of nlap planes of [n][M] (lap may be null:
+// T = w * pot * phi, or with pot null: T = w * phi)
 __global__ void k_weighted_op(int n, int64_t M, const double *__restrict__ w, const double *__restrict__ pot,
-                              const double *__restrict__ phi, const double *__restrict__ lap, double a,
+                              const double *__restrict__ phi, const double *__restrict__ lap, int nlap, double a,
                               double *__restrict__ T) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= (int64_t)n * M) return;
     const int64_t k = e % M;
     double v = pot ? pot[k] * phi[e] : phi[e];
-    if (lap) v += a * lap[e];
+    if (lap) {
+        double l = lap[e];
+        for (int q = 1; q < nlap; ++q) l += lap[(int64_t)q * n * M + e];
+        v += a * l;
+    }
     T[e] = w[k] * v;
 }
 void launch_weighted_op(int n, int64_t M, const double *w, const double *pot, const double *phi, const double *lap,
-                        double a, double *T, hipStream_t s) {
+                        int nlap, double a, double *T, hipStream_t s) {
     const int64_t cnt = (int64_t)n * M;
     if (cnt <= 0) return;
-    hipLaunchKernelGGL(k_weighted_op, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, n, M, w, pot, phi, lap, a,
+    hipLaunchKernelGGL(k_weighted_op, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, n, M, w, pot, phi, lap, nlap, a,
                        T);
 }
 
