@@ -165,7 +165,7 @@ struct flosic_ctx {
     DevBuf<double> d_ps_coef;
     DevBuf<PairDev> d_pairs;
     DevBuf<ChunkDev> d_chunks_bf16;
-    int nchunks_bf16 = 0;
+    int nchunks_bf16 = 0, rgc_bf16[5] = {0, 0, 0, 0, 0};  // chunks and the four runs of them (CoulJob)
     int64_t rows_padded = 0, rows_padded_bf16 = 0;  // Hermite rows as the FP and the split-BF16 kernels stream them
     DevBuf<double> d_lapplane, d_lap, d_pot, d_wop, d_small, d_B, d_hao;  // LAGMULT_SLV / AO SIC Hamiltonian
     DevBuf<double> d_scf;  // SCFSICW orbital update: ham_ao, ham_ao C, C^T ham_ao C
@@ -203,7 +203,7 @@ struct flosic_ctx {
     Spin sp[2];
     // evaluation buffers
     int nF = 0, ldh = 0;  // ldh: nF rounded up to the widest column block (the legal block widths divide it)
-    int ldc = 0;          // leading dimension of H: nF rounded up to 16, ldh for the split-BF16 forms
+    int ldc = 0;          // leading dimension of H: nF rounded up to 16
     DevBuf<double> d_fodxyz, d_fodchi;  // FOD coordinates of both spins (x, y, z arrays), basis planes at them
     DevBuf<double> d_cflo, d_dps, d_H, d_phi, d_VH, d_Vtot, d_U, d_part, d_energy, d_G, d_Gpart, d_vabpart, d_vab,
         d_lambda, d_asy, d_Ux, d_lamex, d_dft, d_dftpart, d_dplanes, d_dphi, d_dvt, d_du, d_dG;
@@ -790,16 +790,19 @@ int build_pairs(flosic_ctx *c) {
                              (p.a * p.A[2] + p.b * p.B[2]) / pe, pe);
     }
     c->nrows = row;
-    // split-BF16 chunk list: consecutive groups of one L, at most `cap_rows` rows, zero-extended to a multiple of `quant`.
+    // split-BF16 chunk list: consecutive groups of one L, at most `cap_rows` rows, zero-extended to that (two K steps).
     // The L = 4 groups (35 rows) go into two chunk types instead: chunk type 5 holds the first 32 rows of two groups,
     // type 6 the last 3 rows of 21 groups; a whole 35-row group would pad its 64-row chunk with 29 zero rows.
     auto make_chunks = [&](int cap_rows, int quant, int64_t &padded) {
         std::vector<ChunkDev> out;
+        int since = 0;
         padded = 0;
         auto emit = [&](int k, int e, int type, int rpg) {
-            const int kr = ((e - k) * rpg + quant - 1) / quant * quant;
-            out.push_back(ChunkDev{k, e, type, kr, pairs[k].row, (int)padded});
-            padded += kr;
+            const int kr = ((e - k) * rpg + quant - 1) / quant * quant;  // what counts towards the next flush
+            since += kr;
+            out.push_back(ChunkDev{k, e, type, cap_rows, pairs[k].row, (int)padded, since >= kFlushRowsBf16});
+            if (out.back().flush) since = 0;
+            padded += cap_rows;
         };
         for (int k = 0; k < c->ngroup;) {
             const int L = pairs[k].lA + pairs[k].lB;
@@ -822,8 +825,14 @@ int build_pairs(flosic_ctx *c) {
         }
         return out;
     };
-    const std::vector<ChunkDev> chunks16 = make_chunks(kChunkRowsBf16, 32, c->rows_padded_bf16);
+    std::vector<ChunkDev> chunks16 = make_chunks(kChunkRowsBf16, 32, c->rows_padded_bf16);
     c->nchunks_bf16 = (int)chunks16.size();
+    if (c->nchunks_bf16 > 0) chunks16.back().flush = 1;
+    c->rgc_bf16[0] = 0;
+    for (int i = 1, k = 0; i < 5; ++i) {  // run i ends after the first flush at or beyond i quarters of the rows
+        while (k < c->nchunks_bf16 && (k == 0 || !chunks16[k - 1].flush || chunks16[k].prow0 < c->rows_padded_bf16 * i / 4)) ++k;
+        c->rgc_bf16[i] = i == 4 ? c->nchunks_bf16 : k;
+    }
     // segment offsets: segL[L] = first group with lA+lB >= L
     for (int L = 0; L <= 5; ++L) {
         int k = 0;
@@ -1038,6 +1047,35 @@ int coulomb_nfb(const flosic_ctx *c) {
     return coulomb_form(c) == COUL_BF16 ? coulomb_cols_split(c->nF) : coulomb_cols(c->nF);
 }
 
+// The Coulomb job of one context in its form, at most nfb columns per block
+template <typename T>
+CoulJob<T> coulomb_job(const flosic_ctx *c, int nfb) {
+    CoulJob<T> J{};
+    const CoulForm form = coulomb_form(c);
+    J.chunks = c->d_chunks_bf16.p;
+    J.nchunks = c->nchunks_bf16;
+    J.seg = c->segL;
+    for (int i = 0; i < 5; ++i) J.rgc[i] = c->rgc_bf16[i];
+    J.pP = c->d_pairP.p;
+    J.H = form == COUL_BF16 ? (const void *)c->d_Hs.p : form == COUL_FP32 ? (const void *)c->d_H32.p
+                                                                           : (const void *)c->d_H64.p;
+    J.nct = c->ldc / 16;
+    J.X = c->d_x.p;
+    J.Y = c->d_y.p;
+    J.Z = c->d_z.p;
+    J.M = c->M;
+    J.nF = c->nF;
+    J.V = c->d_VH.p;
+    J.ldv = c->M;
+    J.nsteps = form == COUL_BF16 ? c->rows_padded_bf16 / 32 : c->rows_padded / 4;
+    J.ncb = coulomb_col_blocks(c->nF, nfb);
+    J.nfb = nfb;
+    const bool far = form == COUL_BF16 && c->prec == FLOSIC_PREC_BF16X3 && c->far_ok && c->far_words > 0;
+    J.far = far ? c->d_far.p : nullptr;
+    J.farw = far ? c->far_words : 0;
+    return J;
+}
+
 // One single-system Coulomb launch of the context's form over M points (x, y, z) into V (ldv), nfb columns
 void coulomb_launch(flosic_ctx *c, const double *x, const double *y, const double *z, int64_t M, double *V,
                     int64_t ldv, int nfb) {
@@ -1048,11 +1086,16 @@ void coulomb_launch(flosic_ctx *c, const double *x, const double *y, const doubl
                            ldv, c->stream);
             break;
         case COUL_BF16: {
+            CoulJob<__bf16> J = coulomb_job<__bf16>(c, nfb);
+            J.X = x;
+            J.Y = y;
+            J.Z = z;
+            J.M = M;
+            J.V = V;
+            J.ldv = ldv;
             // the far bits describe the tiles of the whole mesh (not the autotuner's point sample)
-            const bool mesh = x == c->d_x.p && M == c->M && c->far_ok && c->far_words > 0;
-            launch_coulomb_bf16(c->prec == FLOSIC_PREC_BF16X3 ? 3 : 2, c->d_chunks_bf16.p, c->nchunks_bf16,
-                                c->rows_padded_bf16 / 32, c->d_pairP.p, c->d_Hs.p, c->ldh, x, y, z, M, c->d_btab.p, nF,
-                                V, ldv, c->stream, nfb, mesh ? c->d_far.p : nullptr, mesh ? c->far_words : 0);
+            if (!(x == c->d_x.p && M == c->M)) J.far = nullptr;
+            launch_coulomb_bf16(c->prec == FLOSIC_PREC_BF16X3 ? 3 : 2, J, c->d_btab.p, c->stream);
             break;
         }
         case COUL_FP32:
@@ -1153,7 +1196,7 @@ int eval_fo(flosic_ctx *c) {
     {
         const int nfb = coulomb_cols(nF);
         c->ldh = (nF + nfb - 1) / nfb * nfb;
-        c->ldc = coulomb_form(c) == COUL_BF16 ? c->ldh : (nF + 15) / 16 * 16;
+        c->ldc = (nF + 15) / 16 * 16;
     }
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipEventRecord(c->ev[EV_START], c->stream));
@@ -1209,8 +1252,8 @@ int eval_hermite(flosic_ctx *c) {
     switch (coulomb_form(c)) {
         case COUL_BF16: {
             const int np = c->prec == FLOSIC_PREC_BF16X3 ? 3 : 2;
-            ALLOC(c, c->d_Hs, (size_t)np * c->ldh * c->rows_padded_bf16);
-            launch_split_h(np, c->d_chunks_bf16.p, c->nchunks_bf16, c->d_H.p, c->ldh, nF, c->rows_padded_bf16 / 32,
+            ALLOC(c, c->d_Hs, (size_t)np * c->ldc * c->rows_padded_bf16);
+            launch_split_h(np, c->d_chunks_bf16.p, c->nchunks_bf16, c->d_H.p, c->ldc, nF, c->rows_padded_bf16 / 32,
                            c->d_Hs.p, c->stream);
             if (np == 3) {
                 const int r = ensure_far(c);
@@ -1516,34 +1559,6 @@ std::vector<uint64_t> batch_sig(const flosic_batch *b) {
     return v;
 }
 
-// The Coulomb job of one context in its form
-CoulJob<double> coulomb_job(const flosic_ctx *c) {
-    CoulJob<double> J{};
-    const CoulForm form = coulomb_form(c);
-    const int nfb = coulomb_nfb(c);
-    J.chunks = c->d_chunks_bf16.p;
-    J.nchunks = c->nchunks_bf16;
-    J.seg = c->segL;
-    J.pP = c->d_pairP.p;
-    J.H = form == COUL_BF16 ? (const void *)c->d_Hs.p : form == COUL_FP32 ? (const void *)c->d_H32.p
-                                                                           : (const void *)c->d_H64.p;
-    J.nct = c->ldc / 16;
-    J.X = c->d_x.p;
-    J.Y = c->d_y.p;
-    J.Z = c->d_z.p;
-    J.M = c->M;
-    J.nF = c->nF;
-    J.V = c->d_VH.p;
-    J.ldv = c->M;
-    J.nsteps = form == COUL_BF16 ? c->rows_padded_bf16 / 32 : c->rows_padded / 4;
-    J.ncb = form == COUL_BF16 ? c->ldh / nfb : fp_col_blocks(c->nF, nfb);
-    J.nfb = nfb;
-    const bool far = form == COUL_BF16 && c->prec == FLOSIC_PREC_BF16X3 && c->far_ok && c->far_words > 0;
-    J.far = far ? c->d_far.p : nullptr;
-    J.farw = far ? c->far_words : 0;
-    return J;
-}
-
 // Classes of equal (form, pieces), each one launch whatever the members' column-block widths; jobs heaviest first
 // (work per item ~ K steps x columns), so that the longest items are dispatched first and the hardware dispatcher
 // balances the tail.  The job records and item offsets go to device memory once per plan.
@@ -1571,7 +1586,7 @@ int build_plan(flosic_batch *b) {
     std::vector<int64_t> offs;
     for (auto &k : b->classes) {
         std::vector<CoulJob<double>> jobs;
-        for (int i : k.members) jobs.push_back(coulomb_job(b->ctxs[i]));
+        for (int i : k.members) jobs.push_back(coulomb_job<double>(b->ctxs[i], coulomb_nfb(b->ctxs[i])));
         std::stable_sort(jobs.begin(), jobs.end(), [](const CoulJob<double> &x, const CoulJob<double> &y) {
             return x.nsteps * x.nfb > y.nsteps * y.nfb;
         });
@@ -1582,7 +1597,7 @@ int build_plan(flosic_batch *b) {
         for (const auto &J : jobs) {
             all.push_back(J);
             offs.push_back(items);
-            items += (J.M + 63) / 64 * J.ncb;
+            items += (k.form == COUL_BF16 ? bf16_items(J.M, J.nct, J.ncb) : (J.M + 63) / 64) * J.ncb;
         }
         offs.push_back(items);
         if (items >= (int64_t)INT32_MAX)
@@ -1783,7 +1798,7 @@ int32_t flosic_create(int32_t device, flosic_ctx **out) {
         delete c;
         return FLOSIC_EDEVICE;
     }
-    std::vector<double> tab((size_t)kBoysTableDoubles);
+    std::vector<double> tab((size_t)kBoysTableDoubles + kZeroDoubles, 0.0);
     boys_table(tab.data());
     if (upload(c, c->d_btab, tab) || hipStreamSynchronize(c->stream) != hipSuccess) {
         delete c;

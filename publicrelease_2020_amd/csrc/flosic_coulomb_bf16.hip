@@ -1,104 +1,40 @@
-// Split-BF16 Coulomb kernels (k_coulomb_ws_bf16 and its batched form) and the far-chunk bits.
+// Split-BF16 Coulomb kernels (k_coulomb_bf16 and its batched form) and the far-chunk bits.
 #include "flosic_device.h"
 
 namespace flosic {
 
-constexpr int kCoulThreads = 1024;  // 16 wavefronts: R waves, copy waves, then 8 consumer waves
-constexpr int kConsumerWave0 = 8;
-// split-BF16: the consumers' FP32 accumulators go into their FP64 sums once at least this many Hermite rows have
-// been accumulated (at chunk ends, and after the last chunk).  On the K=64 workload (same box): every 64 rows
-// 1109 ms, 128 rows 1083 ms, 256 rows 1060-1070 ms, 512 rows 1053 ms, with |dE| against FP64 of 4.9e-7, 5.3e-7,
-// 4.4e-7 and 6.2e-7 Ha; the flush (24 FP64 conversions and adds per consumer lane) is VALU work that the kernel's
-// sub-steps wait for.  (The FP32 MFMA form keeps its flush per chunk: every 256 rows saved it under 1% there.)
-constexpr int kFlushRowsBf16 = 256;
-constexpr int kSlotsReg = 2;  // split-BF16: H staged through the copy waves' registers, the sub-step in use and the next
-
-// position in the chunk / sub-step sequence
-struct SubStep {
-    int c, q;
-};
-__device__ __forceinline__ void advance(SubStep &p, const ChunkDev *chunks, int sr) {
-    if (++p.q * sr >= chunk_at(chunks, p.c).kr) {
-        p.q = 0;
-        ++p.c;
-    }
-}
-
-// R of the groups [np*q/nq, np*(q+1)/nq) of chunk `ch` (share q of nq) for the block's 64 points: R wave rw of
-// nrw takes every nrw-th group (wave-uniform, so the group's centre and exponent are scalar loads) and lane l
-// the point k0 + l, whose coordinates (px, py, pz) stay in registers.  LAYOUT 0: Rl[row * LD + point] in T;
-// LAYOUT 2: Rl[point * LD + row] in T.  Share 0 also zeroes the rows beyond the groups.
-// R is computed in FP64 for the FP64 form and in FP32 for the FP32 and split-BF16 operands, with the Boys table of
-// that precision (the FP32 copy follows the FP64 table in device memory; the split-BF16 kernel reads it from LDS)
-// RPG rows per group from Hermite row ROFF on (the whole group by default; the split-BF16 list's L = 4 head / tail
-// chunks take rows [0, 32) / [32, 35) of each group, see chunk_rpg)
-template <int L, typename T, int LD, int LAYOUT, int NP, int RPG = ntuv(L), int ROFF = 0>
-__device__ __forceinline__ void chunk_R(int rw, int nrw, int lane, double px, double py, double pz, bool valid, int q,
-                                        int nq, const ChunkDev &ch, const double4 *__restrict__ pP,
-                                        const RType<T> *__restrict__ ctab, T *Rl) {
-    constexpr int nt = ntuv(L);
-    static_assert(ROFF + RPG <= nt, "chunk rows beyond the group's Hermite block");
-    using C = RType<T>;
-    const int np = ch.pe - ch.pb;
-    const int glo = np * q / nq, ghi = np * (q + 1) / nq;
-    for (int g = glo + rw; g < ghi; g += nrw) {
-        const v4d P = gload(reinterpret_cast<const v4d *>(pP + ch.pb + g));  // x, y, z, p
-        // lanes past the mesh end (valid false, coordinates 0) compute finite values too: an A row feeds only its own
-        // point's output row, which is never stored, so no lane needs its R zeroed (that took nt moves per group)
-        C R[nt];
-        hermite_R<L, C>((C)P.w, (C)(P.x - px), (C)(P.y - py), (C)(P.z - pz), ctab, R);
-#pragma unroll
-        for (int t = 0; t < RPG; ++t) {
-            if constexpr (LAYOUT == 0)
-                Rl[(g * RPG + t) * LD + lane] = (T)R[ROFF + t];
-            else
-                Rl[lane * LD + g * RPG + t] = (T)R[ROFF + t];
-        }
-    }
-    if (q == 0)
-        for (int r = np * RPG + rw; r < ch.kr; r += nrw) {
-            if constexpr (LAYOUT == 0)
-                Rl[r * LD + lane] = (T)0;
-            else
-                Rl[lane * LD + r] = (T)0;
-        }
-}
-
-template <typename T, int LD, int LAYOUT, int NP>
-__device__ __forceinline__ void produce_R(int rw, int nrw, int lane, double px, double py, double pz, bool valid,
-                                          int q, int nq, const ChunkDev &ch, const double4 *__restrict__ pP,
-                                          const RType<T> *__restrict__ tab, T *Rl) {
-    switch (ch.L) {
-        case 0: chunk_R<0, T, LD, LAYOUT, NP>(rw, nrw, lane, px, py, pz, valid, q, nq, ch, pP, tab, Rl); break;
-        case 1: chunk_R<1, T, LD, LAYOUT, NP>(rw, nrw, lane, px, py, pz, valid, q, nq, ch, pP, tab, Rl); break;
-        case 2: chunk_R<2, T, LD, LAYOUT, NP>(rw, nrw, lane, px, py, pz, valid, q, nq, ch, pP, tab, Rl); break;
-        case 3: chunk_R<3, T, LD, LAYOUT, NP>(rw, nrw, lane, px, py, pz, valid, q, nq, ch, pP, tab, Rl); break;
-        case 4: chunk_R<4, T, LD, LAYOUT, NP>(rw, nrw, lane, px, py, pz, valid, q, nq, ch, pP, tab, Rl); break;
-        case 5:
-            chunk_R<4, T, LD, LAYOUT, NP, chunk_rpg(5), chunk_roff(5)>(rw, nrw, lane, px, py, pz, valid, q, nq, ch, pP,
-                                                                      tab, Rl);
-            break;
-        default:
-            chunk_R<4, T, LD, LAYOUT, NP, chunk_rpg(6), chunk_roff(6)>(rw, nrw, lane, px, py, pz, valid, q, nq, ch, pP,
-                                                                      tab, Rl);
-            break;
-    }
-}
-
-// s_waitcnt lgkmcnt(0) alone (vmcnt 63, expcnt 7)
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xF | (7 << 4) | (0 << 8) | (3 << 14)); }
-
 // ---------------------------------------------------------------------------------------------------
 // Split-BF16 Coulomb.  x = x1 + x2 (+ x3) in bf16 pieces, so the product x*y is carried by x1y1 + x1y2 + x2y1
 // (+ x1y3 + x2y2 + x3y1) at ~2^-16 (2^-24) relative error, every term on the 16x16x32 bf16 MFMA (lane l holds
-// A[l%16][8*(l/16) .. +7], B[8*(l/16) .. +7][l%16]; FP32 register r holds D[4*(l/16) + r][l%16]).  Same block
-// organisation as k_coulomb_ws with one 32-row K step per sub-step and consumer waves of 16 points x half the
-// columns.  R is kept in LDS as FP32 [point][row]; each consumer splits its 8-row A operand when it loads it; H
-// pieces come from k_split_h in operand order.  The copy waves stage H through their registers (ordinary 16-byte
-// loads one sub-step ahead, 16-byte LDS stores into two slots): on the 36 KiB split-BF16 sub-steps this moves H
-// faster than the asynchronous global->LDS loads of the FP kernels, which remain faster for their 24 KiB steps.
+// A[l%16][8*(l/16) .. +7], B[8*(l/16) .. +7][l%16]; FP32 register r holds D[4*(l/16) + r][l%16]).
+//
+// Bound.  Per 32 Hermite rows and 64 points: 4 * 6 MFMAs of 16 cycles for every 16 columns against, once, R of the rows'
+// groups (60-110 FP32 VALU instructions per group) and its split into pieces (176 VALU instructions).  Beside bf16 MFMAs
+// FP32 VALU work overlaps only in part (measured: about a quarter of the shorter of the two), so R and the split are made
+// once per 64 points and never again per column: a wave holds 64 points x NT <= 3 tiles of 16 columns (48 FP32
+// accumulators and 48 FP64 sums), and its H operands come from L1/L2 straight into registers.
+//
+// Split.  Block = 8 wavefronts, one block per CU (256 registers per lane).
+//   up to  48 FLOs  CW = 1: two tiles of 64 points; the four waves of a tile hold all its columns, make R and the split
+//                   by themselves for four runs of chunks, and meet in the final sum.  No barrier in the loop.
+//   up to  96 FLOs  CW = 2: two tiles of 64 points; up to 192 FLOs CW = 4: one tile.  More FLOs: further blocks.
+// With CW > 1 the waves have roles, because the sums leave no room for both R and H operands loaded ahead (waves that did
+// everything in turn ran 192 FLOs, 5.2e5 rows, 2.0e5 points at 272 ms, the registers spilling, against 210 ms with roles):
+// waves 0-3 are consumers, CW on each tile, whose H operands are loaded one K step ahead; waves 4-7 producers, CW on each
+// tile.  While the consumers run the MFMAs of chunk c, the producers split R of chunk c + 1 into A operands and make R of
+// chunk c + 2 (FP32, lane = point), both in two LDS buffers; one barrier per chunk of 64 Hermite rows.
+// The FP32 accumulators go into the FP64 sums at the chunks marked flush (every 256 or more rows), so the sums do not
+// depend on the split.
+// Measured, three pieces, against 16-wave blocks in which two waves of every block staged H through LDS: 10 FLOs (289 groups,
+// 3.4e4 points) 0.279 -> 0.126 ms; 30 FLOs (1686, 1.2e5) 2.98 -> 1.24; 48 FLOs (4163, 1.9e5) 12.6 -> 5.5; 64 FLOs (7371,
+// 2.4e5) 25.8 -> 20.5; 96 FLOs (15750, 3.7e5) 96.0 -> 76.2; 120 FLOs (24241, 3.1e5) 104 -> 93.7; 144 FLOs (33810, 2.8e5)
+// 162 -> 121; 192 FLOs (60795, 2.0e5) 242 -> 210.  With CW = 1 making R bounds the loop (32 and 48 FLOs take the same time per
+// row and point); with CW = 4 the MFMAs are 52% busy, producers alone take 140 ms of the 210 and consumers alone 170.
 // ---------------------------------------------------------------------------------------------------
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef unsigned v4w __attribute__((ext_vector_type(4)));
 
 template <int NP>
 __device__ __forceinline__ void split_bf16(double x, __bf16 *out, int64_t stride) {
@@ -204,271 +140,506 @@ void launch_far_bits(const double *x, const double *y, const double *z, int64_t 
 // remainder of the previous ones, so that the pieces shrink by 2^-8 each and the last remainder is below 2^-8 of
 // the last piece.  (An exact split by truncation, keeping the upper 16 bits of each remainder, is 1% faster here
 // but its pieces shrink only by 2^-7, which triples the worst dropped cross product.)
-// Rows go two at a time through one packed conversion (v_cvt_pk_bf16_f32, round to nearest even like the scalar
-// cast); a piece's bf16 value is back in FP32 by a shift (low half) or a mask (high half) of the packed word, so a
-// piece of two rows costs 5 VALU operations and the split needs no repacking into the operand vector.
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef unsigned v4w __attribute__((ext_vector_type(4)));
+// Rows go two at a time through one packed conversion (v_cvt_pk_bf16_f32, round to nearest even like the scalar cast);
+// v_dot2_f32_bf16 with (-1, 0) or (0, -1) subtracts one half of the packed word from its row (an exact difference: checked
+// bit for bit against the FP32 subtraction over 2^-149 .. 2^40), so a piece of two rows costs 3 VALU operations, where
+// shift, mask and two subtractions would make it 5.  The constants go through registers: as an inline constant -1.0 they
+// would be read as one 32-bit value.
 template <int NP>
-__device__ __forceinline__ void split_a(const float *src, v8bf (&a)[NP]) {
-    const v4f x0 = *(const v4f *)src, x1 = *(const v4f *)(src + 4);
+__device__ __forceinline__ void split_a(v4f x0, v4f x1, v8bf (&a)[NP]) {
     float r[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+    unsigned lo = 0x0000bf80u, hi = 0xbf800000u;
+    asm("" : "+s"(lo), "+s"(hi));
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         v4w w;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){r[2 * e], r[2 * e + 1]}, v2bf));
-            w[e] = u;
+            const v2bf u = __builtin_convertvector((v2f){r[2 * e], r[2 * e + 1]}, v2bf);
+            w[e] = __builtin_bit_cast(unsigned, u);
             if (p + 1 < NP) {
-                r[2 * e] -= __builtin_bit_cast(float, u << 16);
-                r[2 * e + 1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+                r[2 * e] = __builtin_amdgcn_fdot2_f32_bf16(u, __builtin_bit_cast(v2bf, lo), r[2 * e], false);
+                r[2 * e + 1] = __builtin_amdgcn_fdot2_f32_bf16(u, __builtin_bit_cast(v2bf, hi), r[2 * e + 1], false);
             }
         }
         a[p] = __builtin_bit_cast(v8bf, w);
     }
 }
 
-// The 1 KiB units (64 lanes x 16 bytes) of one staged K step that copy wave cw of NCPW moves, through registers:
-// unit u = pc * NFB/16 + v is KiB v of piece pc's run for the block's columns, at LDS slot offset u KiB.
-template <int NP, int NFB, int NCPW>
-struct HUnits {
-    static constexpr int UPP = NFB / 16, NU = NP * UPP, UPW = (NU + NCPW - 1) / NCPW;
-    typedef unsigned v4u __attribute__((ext_vector_type(4)));
-    v4u r[UPW];
-    // the units of the sub-step whose piece-0 run for the block's columns starts at sub_base, the pieces pstride bytes
-    // apart; npe: pieces read from H (NP, or 2 for a far chunk, whose third piece is staged as zeros)
-    __device__ __forceinline__ void load_at(const char *sub_base, int64_t pstride, int cw, int lane, int npe) {
+// R of a chunk in LDS: 64 rows of 64 points in FP32.  PAD: 68 floats per point (16-byte accesses free of conflicts, offsets
+// inside a group immediate); else 64 floats per point whose 16-byte slots are permuted by the point (CW = 2, where the
+// padding does not fit).
+template <bool PAD>
+constexpr int bf_rsize = 64 * (PAD ? 68 : 64);
+template <bool PAD>
+__device__ __forceinline__ int r_at(int point, int row) {
+    return PAD ? point * 68 + row : point * 64 + (((row >> 2) ^ (point & 15)) << 2) + (row & 3);
+}
+
+template <int NP, int CW>
+struct BfTile {                         // LDS of one 64-point tile with CW > 1
+    float R[2][bf_rsize<CW == 4>];
+    v8bf A[2][2][4][NP][64];            // A operands [buffer][K step][point tile][piece][lane]
+};
+constexpr int kBfTab = kBoysRows * kBoysCols * 4;  // the FP32 Boys table, in LDS with CW = 4
+template <int NP, int CW>
+constexpr int bf_lds = CW == 1 ? 8 * bf_rsize<true> * 4 : (4 / CW) * (int)sizeof(BfTile<NP, CW>) + (CW == 4 ? kBfTab : 0);
+template <int NP>
+constexpr int bf_lds_all = bf_lds<NP, 1> > bf_lds<NP, 2> && bf_lds<NP, 1> > bf_lds<NP, 4> ? bf_lds<NP, 1>
+                           : bf_lds<NP, 2> > bf_lds<NP, 4>                                ? bf_lds<NP, 2>
+                                                                                          : bf_lds<NP, 4>;
+constexpr int kBfOut = 16 * 66;  // one column tile of FP64 sums in the epilogue, per wave
+
+// hermite_R<L, float> of NG groups at once: the same operations, ordered so that two groups' chains overlap.  The far branch
+// of the Boys functions (12 VALU instructions) is taken by every lane, the near one (table) if a lane of the wave needs it.
+// TAIL: only the last three rows of L = 4, R_022, R_013 and R_004 (chunk type 6), which need 15 of the 65 steps.
+template <int L, int NG, bool TAIL>
+__device__ __forceinline__ void hermite_Rn(const float *p, const float (*X)[3], const float *__restrict__ tab,
+                                           float (*R)[ntuv(L)]) {
+    constexpr int TOP = L < 2 ? 2 : L;
+    float T[NG], eT[NG], F[NG][TOP + 1];
 #pragma unroll
-        for (int k = 0; k < UPW; ++k) {
-            const int u = cw + k * NCPW;
-            if (u < npe * UPP) {
-                const int pc = u / UPP, v = u - pc * UPP;
-                r[k] = gload((const v4u *)(sub_base + pc * pstride + v * 1024 + lane * 16));
-            } else if (u < NU) {
-                r[k] = v4u{0u, 0u, 0u, 0u};
-            }
+    for (int g = 0; g < NG; ++g) {
+        T[g] = p[g] * __builtin_fmaf(X[g][2], X[g][2], __builtin_fmaf(X[g][0], X[g][0], X[g][1] * X[g][1]));
+        eT[g] = __expf(-T[g]);
+        boys32_far<TOP>(T[g], eT[g], F[g]);
+    }
+    if (__any(!(T[0] > 16.0f) || !(T[NG - 1] > 16.0f))) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const bool far = T[g] > 16.0f;
+            float N[TOP + 1];
+            boys32_near<TOP>(far ? 0.0f : T[g], eT[g], tab, N);
+#pragma unroll
+            for (int m = 0; m <= TOP; ++m) F[g][m] = far ? F[g][m] : N[m];
         }
     }
-    __device__ __forceinline__ void store(__bf16 *slot, int cw, int lane) const {
 #pragma unroll
-        for (int k = 0; k < UPW; ++k) {
-            const int u = cw + k * NCPW;
-            if (u < NU) *(v4u *)((char *)slot + u * 1024 + lane * 16) = r[k];
+    for (int g = 0; g < NG; ++g) {
+        float pw[L + 1];
+        pw[0] = 1.0f;
+#pragma unroll
+        for (int n = 1; n <= L; ++n) pw[n] = pw[n - 1] * (-2.0f * p[g]);
+        if constexpr (TAIL) {
+            const float Y = X[g][1], Z = X[g][2];
+            const float a = pw[3] * F[g][3], b = a * Z;                          // R_000 of level 3, R_001 of level 2
+            const float d = __builtin_fmaf(pw[4] * F[g][4] * Z, Z, a);           // R_002 of level 2
+            const float e = __builtin_fmaf(2.0f, b, d * Z);                      // R_003 of level 1
+            const float f = __builtin_fmaf(pw[2], F[g][2], b * Z);               // R_002 of level 1
+            R[g][32] = __builtin_fmaf(d * Y, Y, f);
+            R[g][33] = e * Y;
+            R[g][34] = __builtin_fmaf(3.0f, f, e * Z);
+        } else {
+            R[g][0] = pw[L] * F[g][L];
+            rlevels<L, L - 1, float>(R[g], X[g][0], X[g][1], X[g][2], F[g], pw);
         }
-    }
-};
-
-// LDS of one split-BF16 Coulomb tile: the two FP32 R tiles, the ring of staged H sub-steps, the FP32 Boys table
-template <int NP, int NFB>
-struct Bf16TileLds {
-    static constexpr int LDK = kChunkRowsBf16 + 4;  // FP32 point rows of 272 bytes: conflict-free 16-byte reads
-    static constexpr int SLOT = NP * NFB * 32;      // bf16 elements of one staged K step
-    __attribute__((aligned(16))) float Rf[2][64 * LDK];
-    __attribute__((aligned(16))) __bf16 Hl[kSlotsReg][SLOT];
-    __attribute__((aligned(16))) float Tb[kBoysRows * kBoysCols];
-    unsigned Fl[NP == 3 ? kFarWords : 1];  // far-chunk bits of this tile (three-piece form)
-};
-
-// One 32-row K step of a consumer wave (16 points x NFB/2 columns): the A operand split into NPE pieces and the
-// products of the pieces down to order 2^-8(NPE-1): 3 (a0b0, a0b1, a1b0) for NPE = 2, plus a0b2, a1b1, a2b0 for
-// NPE = 3 (zero for a0b2 in a far chunk, whose staged third H piece is zero)
-template <int NPE, int NFB>
-__device__ __forceinline__ void bf16_substep(const float *Rrow, const __bf16 *Hs_, int cl0, int lane,
-                                             v4f (&acc)[NFB / 32]) {
-    v8bf a[NPE];
-    split_a<NPE>(Rrow, a);
-#pragma unroll
-    for (int j = 0; j < NFB / 32; ++j) {
-        v8bf b[NPE];
-#pragma unroll
-        for (int p = 0; p < NPE; ++p) b[p] = *(const v8bf *)(Hs_ + ((p * (NFB / 16) + cl0 + j) * 64 + lane) * 8);
-        v4f cc = acc[j];
-        cc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], cc, 0, 0, 0);
-        cc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], cc, 0, 0, 0);
-        cc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], cc, 0, 0, 0);
-        if constexpr (NPE == 3) {
-            cc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], cc, 0, 0, 0);
-            cc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], cc, 0, 0, 0);
-            cc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], cc, 0, 0, 0);
-        }
-        acc[j] = cc;
     }
 }
 
-// far: null, or the far-chunk bits of every tile (farw 32-bit words per tile, bit c of a tile's row set where every
-// (point, group) pair of tile and chunk c has T = p|r - P|^2 above the far threshold): the three-piece form reads
-// two H pieces of those chunks from memory and stages the third as zeros (H to ~2^-17 there, R still in three)
-template <int NP, int NFB>
-__device__ __forceinline__ void coulomb_tile_bf16(Bf16TileLds<NP, NFB> &L, const ChunkDev *__restrict__ chunks,
-                                                  int nchunks, int64_t nsteps,
-                                                  const double4 *__restrict__ pP, const __bf16 *__restrict__ Hs,
-                                                  int nct, const double *__restrict__ X, const double *__restrict__ Y,
-                                                  const double *__restrict__ Z, int64_t M, int nF,
-                                                  double *__restrict__ V, int64_t ldv,
-                                                  const double *__restrict__ tab, int64_t tile, int cb,
-                                                  const unsigned *__restrict__ far, int farw) {
-    constexpr int TP = 64, NCW = NFB / 32, SR = 32;  // consumer wave: 16 points x NFB/2 columns
-    constexpr int NCPW = NP == 3 ? 2 : 1, NRW = kConsumerWave0 - NCPW;
-    constexpr int LDK = Bf16TileLds<NP, NFB>::LDK;
-    constexpr int SLOT = Bf16TileLds<NP, NFB>::SLOT;
-    float(&Rf)[2][TP * LDK] = L.Rf;
-    __bf16(&Hl)[kSlotsReg][SLOT] = L.Hl;
-    float(&Tb)[kBoysRows * kBoysCols] = L.Tb;  // FP32 Boys table for the R waves
-    const int64_t k0 = tile * TP;
-    const int fb = cb * NFB;
-    // the wave index through readfirstlane: the compiler then knows it (and every role, group, unit and tile index
-    // derived from it) to be wave-uniform and keeps that arithmetic and the load addresses built on it scalar
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const bool use_far = NP == 3 && far != nullptr;
-    {  // the table in LDS keeps the R waves' per-lane table lookups off the load path of the H copies
-        const v4f *src = (const v4f *)(tab + kBoysRows * kBoysCols);
-        for (int i = threadIdx.x; i < kBoysRows * kBoysCols / 4; i += kCoulThreads) ((v4f *)Tb)[i] = src[i];
-        if (use_far)
-            for (int i = threadIdx.x; i < farw; i += kCoulThreads) L.Fl[i] = gload(far + tile * farw + i);
+// R of NG groups of a chunk, g0 and g0 + step (rows RPG g .. of the chunk hold rows ROFF .. of group g), for this lane's
+// point
+template <bool PAD, int L, int RPG, int ROFF, int NG>
+__device__ __forceinline__ void bf_groups(const double4 *__restrict__ pP, int g0, int step, int lane, double px, double py,
+                                          double pz, const float *__restrict__ tab, float *__restrict__ R) {
+    float p[NG], X[NG][3], r[NG][ntuv(L)];
+#pragma unroll
+    for (int e = 0; e < NG; ++e) {
+        const v4d P = cload(reinterpret_cast<const v4d *>(pP + g0 + e * step));
+        p[e] = (float)P.w;
+        X[e][0] = (float)(P.x - px);
+        X[e][1] = (float)(P.y - py);
+        X[e][2] = (float)(P.z - pz);
+    }
+    hermite_Rn<L, NG, ROFF == 32>(p, X, tab, r);
+#pragma unroll
+    for (int e = 0; e < NG; ++e) {
+        const int row0 = (g0 + e * step) * RPG;
+        if constexpr (RPG % 4 == 0) {
+#pragma unroll
+            for (int t = 0; t < RPG; t += 4)
+                *(v4f *)(R + r_at<PAD>(lane, row0 + t)) =
+                    v4f{r[e][ROFF + t], r[e][ROFF + t + 1], r[e][ROFF + t + 2], r[e][ROFF + t + 3]};
+        } else if constexpr (RPG % 2 == 0) {
+#pragma unroll
+            for (int t = 0; t < RPG; t += 2) *(v2f *)(R + r_at<PAD>(lane, row0 + t)) = v2f{r[e][ROFF + t], r[e][ROFF + t + 1]};
+        } else {
+#pragma unroll
+            for (int t = 0; t < RPG; ++t) R[r_at<PAD>(lane, row0 + t)] = r[e][ROFF + t];
+        }
+    }
+}
+// groups first, first + step, ... of the chunk, two at a time
+template <bool PAD, int L, int RPG = ntuv(L), int ROFF = 0>
+__device__ __forceinline__ void bf_chunk_R(const ChunkDev &ch, int first, int step, const double4 *__restrict__ pP,
+                                           int lane, double px, double py, double pz, const float *__restrict__ tab,
+                                           float *__restrict__ R) {
+    const int np = ch.pe - ch.pb;
+    int g = first;
+    for (; g + step < np; g += 2 * step)
+        bf_groups<PAD, L, RPG, ROFF, 2>(pP + ch.pb, g, step, lane, px, py, pz, tab, R);
+    if (g < np) bf_groups<PAD, L, RPG, ROFF, 1>(pP + ch.pb, g, step, lane, px, py, pz, tab, R);
+}
+
+template <bool PAD>
+__device__ __forceinline__ void bf_make_R(const ChunkDev &ch, int first, int step, const double4 *__restrict__ pP, int lane,
+                                          double px, double py, double pz, const float *__restrict__ tab,
+                                          float *__restrict__ R) {
+    switch (ch.L) {
+        case 0: bf_chunk_R<PAD, 0>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
+        case 1: bf_chunk_R<PAD, 1>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
+        case 2: bf_chunk_R<PAD, 2>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
+        case 3: bf_chunk_R<PAD, 3>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
+        case 5: bf_chunk_R<PAD, 4, chunk_rpg(5), chunk_roff(5)>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
+        default: bf_chunk_R<PAD, 4, chunk_rpg(6), chunk_roff(6)>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
+    }
+}
+// rows 32 q + 8 lr .. + 7 of point 16 i + lc, split
+template <int NP, bool PAD>
+__device__ __forceinline__ void bf_rows8(const float *R, int i, int q, int lr, int lc, v8bf (&a)[NP]) {
+    const int pt = 16 * i + lc, row = 32 * q + 8 * lr;
+    split_a<NP>(*(const v4f *)(R + r_at<PAD>(pt, row)), *(const v4f *)(R + r_at<PAD>(pt, row + 4)), a);
+}
+
+template <int NP, int NT>
+struct BfAcc {
+    v4f acc[4][NT];
+    double sum[4][NT][4];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    acc[i][j][r] = 0.0f;
+                    sum[i][j][r] = 0.0;
+                }
+    }
+    __device__ __forceinline__ void flush() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    sum[i][j][r] += (double)acc[i][j][r];
+                    acc[i][j][r] = 0.0f;
+                }
+    }
+    // one K step: products of the pieces in the order a0b0, a0b1, a1b0 (a0b2, a1b1, a2b0) for every accumulator, one point
+    // tile after the other.  next_a(i, a) gives the A operand of tile i; it is issued before the MFMAs of tile i - 1 and,
+    // with HOLD, the scheduler is kept from moving it down to its use.
+    template <bool HOLD, typename F>
+    __device__ __forceinline__ void step(F next_a, const v8bf (&b)[NT][NP]) {
+        v8bf a[2][NP];
+        next_a(0, a[0]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i < 3) next_a(i + 1, a[(i + 1) & 1]);
+            if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);
+#define FLOSIC_BF(pa, pb)                          \
+    _Pragma("unroll") for (int j = 0; j < NT; ++j) \
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i & 1][pa], b[j][pb], acc[i][j], 0, 0, 0)
+            FLOSIC_BF(0, 0);
+            FLOSIC_BF(0, 1);
+            FLOSIC_BF(1, 0);
+            if constexpr (NP == 3) {
+                FLOSIC_BF(0, 2);
+                FLOSIC_BF(1, 1);
+                FLOSIC_BF(2, 0);
+            }
+#undef FLOSIC_BF
+            if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+};
+// B operands of the K step at h (piece 0 of this wave's first column tile).  In a far chunk the third piece counts as zero:
+// it is loaded from `zero` (this lane's place in a run of zeros), so that every K step issues the same loads and the waits
+// for them can be counted.
+template <int NP, int NT>
+__device__ __forceinline__ void bf_load(v8bf (&b)[NT][NP], const char *h, int64_t pstride, bool far, const char *zero) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const char *src = p == 2 && far ? zero : h + p * pstride;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) b[j][p] = gload((const v8bf *)(src + j * 1024));
+    }
+}
+template <int NP>
+__device__ __forceinline__ bool bf_far(const unsigned *far, int c) {  // far: this tile's chunk bits, or null
+    if (NP != 3 || !far) return false;
+    return (__builtin_amdgcn_readfirstlane(cload(far + (c >> 5))) >> (c & 31)) & 1u;
+}
+
+// Barrier between producers and consumers: this wave's LDS accesses are done, its global loads stay in flight (the fence
+// of __syncthreads would wait for them)
+__device__ __forceinline__ void role_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    wait_lgkm0();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Epilogue: one column tile of sums at a time through LDS, [column][66 points]: 512 contiguous bytes per store.  With
+// CW = 1 the four row groups of a tile are added there and each stores four columns.
+template <int NP, int CW, int NT>
+__device__ __forceinline__ void bf_store(unsigned char *__restrict__ lds, const CoulJob<__bf16> &J, const BfAcc<NP, NT> &A,
+                                         int64_t kl, bool valid, int wave, int ct0, int ntmax) {
+    constexpr int RW = CW == 1 ? 4 : 1;
+    const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15, rg = wave % RW, w0 = wave - rg;
+    double *o = reinterpret_cast<double *>(lds);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        if (j >= ntmax) break;
+        __syncthreads();
+        if (j < NT) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    o[wave * kBfOut + lc * 66 + i * 16 + 4 * lr + r] = A.sum[i][j < NT ? j : 0][r];
+        }
+        __syncthreads();
+        if (j < NT) {
+#pragma unroll
+            for (int q = 0; q < 16 / RW; ++q) {
+                const int col = rg * (16 / RW) + q, f = (ct0 + j) * 16 + col;
+                double v = o[w0 * kBfOut + col * 66 + lane];
+#pragma unroll
+                for (int g = 1; g < RW; ++g) v += o[(w0 + g) * kBfOut + col * 66 + lane];
+                if (f < J.nF && valid) gstore(J.V + (int64_t)f * J.ldv + kl, v);
+            }
+        }
+    }
+}
+
+// this lane's point of a tile
+struct BfPoint {
+    int64_t k;
+    bool valid;
+    double x, y, z;
+};
+__device__ __forceinline__ BfPoint bf_point(const CoulJob<__bf16> &J, int64_t tile) {
+    BfPoint p;
+    p.k = tile * 64 + (threadIdx.x & 63);
+    p.valid = p.k < J.M;
+    p.x = p.valid ? gload(J.X + p.k) : 0.0;
+    p.y = p.valid ? gload(J.Y + p.k) : 0.0;
+    p.z = p.valid ? gload(J.Z + p.k) : 0.0;
+    return p;
+}
+__device__ __forceinline__ const unsigned *bf_far_row(const CoulJob<__bf16> &J, int64_t tile) {
+    return J.far && tile * 64 < J.M ? J.far + tile * J.farw : nullptr;
+}
+
+// CW = 1: a wave on its own run of chunks, all columns
+template <int NP, int NT>
+__device__ __forceinline__ void bf_alone(unsigned char *__restrict__ lds, const CoulJob<__bf16> &J,
+                                         const double *__restrict__ tab, int64_t tile, int wave, int ct0) {
+    const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15, rg = wave % 4;
+    const BfPoint P = bf_point(J, tile);
+    const float *ctab = (const float *)(tab + kBoysRows * kBoysCols);
+    const char *zero = (const char *)(tab + kBoysTableDoubles) + lane * 16;
+    float *R = reinterpret_cast<float *>(lds) + wave * bf_rsize<true>;
+    const int c0 = J.rgc[rg], c1 = J.rgc[rg + 1];
+    const unsigned *far = bf_far_row(J, tile);
+    // rows of a chunk beyond its groups are never written and meet zero rows of H: they only have to be finite
+    for (int i = lane; i < bf_rsize<true> / 4; i += 64) ((v4f *)R)[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    wave_lds_sync();
+    BfAcc<NP, NT> A;
+    A.clear();
+    const int64_t pstride = J.nsteps * J.nct * 1024, hstep = (int64_t)J.nct * 1024;
+    const char *h = (const char *)J.H + ((int64_t)ct0 * 64 + lane) * 16;  // piece 0 of the next K step to be loaded
+    v8bf b[NT][NP];
+    if (c0 < c1) {
+        h += (int64_t)(chunk_at(J.chunks, c0).prow0 / 32) * hstep;
+        bf_load<NP, NT>(b, h, pstride, bf_far<NP>(far, c0), zero);
+    }
+    for (int c = c0; c < c1;) {
+        int flush;
+        do {
+        const ChunkDev ch = chunk_at(J.chunks, c);
+        bf_make_R<true>(ch, 0, 1, J.pP, lane, P.x, P.y, P.z, ctab, R);
+        wave_lds_sync();
+        const bool f = bf_far<NP>(far, c);
+#pragma unroll 1
+        for (int q = 0; q < 2; ++q) {
+            auto next_a = [&](int i, v8bf(&a)[NP]) { bf_rows8<NP, true>(R, i, q, lr, lc, a); };
+            A.template step<true>(next_a, b);
+            h += hstep;
+            if (q == 0) bf_load<NP, NT>(b, h, pstride, f, zero);
+            else if (c + 1 < c1) bf_load<NP, NT>(b, h, pstride, bf_far<NP>(far, c + 1), zero);
+        }
+        flush = ch.flush;
+        ++c;
+        wave_lds_sync();
+        } while (!flush);
+        A.flush();
+    }
+    bf_store<NP, 1, NT>(lds, J, A, P.k, P.valid, wave, ct0, NT);
+}
+
+template <int NP, int CW>
+__device__ __forceinline__ void bf_producer(BfTile<NP, CW> &T, const CoulJob<__bf16> &J, const float *__restrict__ ctab,
+                                            int64_t tile, int pi, int ntmax) {
+    const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15;
+    const BfPoint P = bf_point(J, tile);
+    const int n = J.nchunks;
+    // rows of a chunk beyond its groups are never written and meet zero rows of H: they only have to be finite
+    for (int i = pi * 64 + lane; i < bf_rsize<CW == 4> / 2; i += 64 * CW) ((v4f *)T.R[0])[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    role_barrier();
+    auto make = [&](int c) {  // which producer begins changes from chunk to chunk
+        bf_make_R<CW == 4>(chunk_at(J.chunks, c), (pi + c) % CW, CW, J.pP, lane, P.x, P.y, P.z, ctab, T.R[c & 1]);
+    };
+    auto split = [&](int c) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int e = 0; e < 4 / CW; ++e) {
+                const int i = pi * (4 / CW) + e;
+                v8bf a[NP];
+                bf_rows8<NP, CW == 4>(T.R[c & 1], i, q, lr, lc, a);
+#pragma unroll
+                for (int p = 0; p < NP; ++p) T.A[c & 1][q][i][p][lane] = a[p];
+            }
+    };
+    make(0);
+    role_barrier();
+    split(0);
+    if (n > 1) make(1);
+    role_barrier();
+    for (int c = 0; c < n; ++c) {
+        if (c + 1 < n) split(c + 1);
+        if (c + 2 < n) make(c + 2);
+        role_barrier();
+    }
+    for (int j = 0; j < ntmax; ++j) {  // the consumers' epilogue
+        __syncthreads();
         __syncthreads();
     }
-    // H pieces read from memory for chunk c (uniform)
-    auto pieces = [&](int c) -> int {
-        if (!use_far) return NP;
-        const unsigned w = __builtin_amdgcn_readfirstlane(L.Fl[c >> 5]);
-        return (w >> (c & 31)) & 1u ? 2 : NP;
-    };
-    if (wave < NRW) {  // R waves: lane l works on point k0 + l throughout
-        const int64_t k = k0 + lane;
-        const bool valid = k < M;
-        const double px = valid ? gload(X + k) : 0.0, py = valid ? gload(Y + k) : 0.0, pz = valid ? gload(Z + k) : 0.0;
-        produce_R<float, LDK, 2, 1>(wave, NRW, lane, px, py, pz, valid, 0, 1, chunk_at(chunks, 0), pP, Tb, Rf[0]);
-        __syncthreads();
-        for (int c = 0; c < nchunks; ++c) {
-            const int nsub = chunk_at(chunks, c).kr / SR;
-            for (int q = 0; q < nsub; ++q) {
-                if (c + 1 < nchunks)
-                    produce_R<float, LDK, 2, 1>(wave, NRW, lane, px, py, pz, valid, q, nsub, chunk_at(chunks, c + 1),
-                                                pP, Tb, Rf[(c + 1) & 1]);
-                __syncthreads();
-            }
+}
+
+template <int NP, int CW, int NT>
+__device__ __forceinline__ void bf_consumer(unsigned char *__restrict__ lds, BfTile<NP, CW> &T, const CoulJob<__bf16> &J,
+                                            const char *zero, int64_t tile, int wave, int ct0, int ntmax) {
+    const int lane = threadIdx.x & 63;
+    const int64_t kl = tile * 64 + lane;
+    const int n = J.nchunks;
+    const unsigned *far = bf_far_row(J, tile);
+    BfAcc<NP, NT> A;
+    A.clear();
+    const int64_t pstride = J.nsteps * J.nct * 1024, hstep = (int64_t)J.nct * 1024;
+    const char *h = (const char *)J.H + ((int64_t)ct0 * 64 + lane) * 16;  // piece 0 of this chunk's first K step
+    v8bf b0[NT][NP], b1[NT][NP];
+    bool f = bf_far<NP>(far, 0);
+    bf_load<NP, NT>(b0, h, pstride, f, zero);
+    bf_load<NP, NT>(b1, h + hstep, pstride, f, zero);
+    __builtin_amdgcn_s_setprio(2);  // MFMAs first, the producer beside them fills the gaps
+    role_barrier();
+    role_barrier();
+    role_barrier();
+    for (int c = 0; c < n;) {
+        int flush;
+        do {  // up to the next flush, which the last chunk has: the sums are not live across a branch
+        const bool more = c + 1 < n, fn = more && bf_far<NP>(far, c + 1);
+        flush = __builtin_amdgcn_readfirstlane(cload(&J.chunks[c].flush));
+        if (more) h += 2 * hstep;  // the last chunk's are loaded again
+        auto a0 = [&](int i, v8bf(&a)[NP]) {
+#pragma unroll
+            for (int p = 0; p < NP; ++p) a[p] = T.A[c & 1][0][i][p][lane];
+        };
+        auto a1 = [&](int i, v8bf(&a)[NP]) {
+#pragma unroll
+            for (int p = 0; p < NP; ++p) a[p] = T.A[c & 1][1][i][p][lane];
+        };
+        A.template step<CW == 4>(a0, b0);
+        bf_load<NP, NT>(b0, h, pstride, fn, zero);
+        A.template step<CW == 4>(a1, b1);
+        bf_load<NP, NT>(b1, h + hstep, pstride, fn, zero);
+        f = fn;
+        ++c;
+        role_barrier();
+        } while (!flush);
+        A.flush();
+    }
+    bf_store<NP, CW, NT>(lds, J, A, kl, kl < J.M, wave, ct0, ntmax);
+}
+
+// Work item `item` of a system: 64-point tiles 2 item and 2 item + 1 (CW = 4: tile item), column block cb of ncb; the
+// column tiles are shared out evenly over the blocks and over a block's column waves
+template <int NP, int CW, int NTLO, int NTHI>
+__device__ __forceinline__ void coulomb_tile_bf16(unsigned char *__restrict__ lds, const CoulJob<__bf16> &J,
+                                                  const double *__restrict__ tab, int64_t item, int cb) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tb0 = J.nct * cb / J.ncb, tb = J.nct * (cb + 1) / J.ncb - tb0;
+    if constexpr (CW == 1) {
+        const int64_t tile = 2 * item + wave / 4;
+        if constexpr (NTHI >= 3) {
+            if (tb == 3) return bf_alone<NP, 3>(lds, J, tab, tile, wave, tb0);
         }
-    } else if (wave < kConsumerWave0) {  // copy waves: H of sub-step gs + 2 is loaded in iteration gs, stored in gs + 1
-        const int cw = wave - NRW;
-        HUnits<NP, NFB, NCPW> h;
-        SubStep nxt{0, 0};
-        // H of sub-step g (chunk c, step q: g = prow0(c) / 32 + q, the sub-steps consecutive in the padded row space)
-        // for the block's columns starts g * nct KiB after hb; the pieces' runs are pstride bytes apart
-        const int64_t pstride = nsteps * nct * 1024;
-        const char *hb = (const char *)(Hs + (fb / 16) * 512);
-        int64_t gnext = 0;  // sub-step index of nxt
-        h.load_at(hb, pstride, cw, lane, pieces(0));
-        h.store(Hl[0], cw, lane);
-        advance(nxt, chunks, SR);
-        ++gnext;
-        bool held = nxt.c < nchunks;  // h holds the next sub-step
-        if (held) {
-            h.load_at(hb + gnext * nct * 1024, pstride, cw, lane, pieces(nxt.c));
-            advance(nxt, chunks, SR);
-            ++gnext;
+        if constexpr (NTLO <= 2 && NTHI >= 2) {
+            if (tb == 2) return bf_alone<NP, 2>(lds, J, tab, tile, wave, tb0);
         }
-        wait_lgkm0();
-        __builtin_amdgcn_s_barrier();
-        int gs = 0;
-        for (int c = 0; c < nchunks; ++c) {
-            const int nsub = chunk_at(chunks, c).kr / SR;
-            for (int q = 0; q < nsub; ++q, ++gs) {
-                if (held) h.store(Hl[(gs + 1) % kSlotsReg], cw, lane);
-                held = nxt.c < nchunks;
-                if (held) {
-                    h.load_at(hb + gnext * nct * 1024, pstride, cw, lane, pieces(nxt.c));
-                    advance(nxt, chunks, SR);
-                    ++gnext;
-                }
-                // the stores must have landed; the loads just issued stay in flight across the barrier
-                wait_lgkm0();
-                __builtin_amdgcn_s_barrier();
-            }
+        if constexpr (NTLO <= 1) {
+            if (tb == 1) return bf_alone<NP, 1>(lds, J, tab, tile, wave, tb0);
         }
     } else {
-    const int cwv = wave - kConsumerWave0;
-    const int lr = lane >> 4, lc = lane & 15;
-    const int pw = (cwv >> 1) * 16;   // point tile of this wave
-    const int cl0 = (cwv & 1) * NCW;  // first column tile of this wave inside the block
-    v4f acc[NCW];
-    double sum[NCW][4];
-#pragma unroll
-    for (int j = 0; j < NCW; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            acc[j][r] = 0.0f;
-            sum[j][r] = 0.0;
-        }
-    __syncthreads();
-    int gs = 0, since = 0;  // since: rows accumulated in FP32 since the last flush into the FP64 sums
-    for (int c = 0; c < nchunks; ++c) {
-        const int kr = chunk_at(chunks, c).kr, nsub = kr / SR;
-        const float *R = Rf[c & 1];
-        since += kr;
-        const bool flush = since >= kFlushRowsBf16 || c + 1 == nchunks;
-        if (flush) since = 0;
-        for (int q = 0; q < nsub; ++q, ++gs) {
-            bf16_substep<NP, NFB>(R + (pw + lc) * LDK + SR * q + 8 * lr, Hl[gs % kSlotsReg], cl0, lane, acc);
-            if (flush && q + 1 == nsub) {
-#pragma unroll
-                for (int j = 0; j < NCW; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        sum[j][r] += (double)acc[j][r];
-                        acc[j][r] = 0.0f;
-                    }
-            }
+        const int w = wave & 3, cw = w % CW, ntmax = (tb + CW - 1) / CW;
+        const int64_t tile = CW == 2 ? 2 * item + w / 2 : item;
+        BfTile<NP, CW> &T = reinterpret_cast<BfTile<NP, CW> *>(lds)[CW == 2 ? w / 2 : 0];
+        const float *ctab = (const float *)(tab + kBoysRows * kBoysCols);
+        if constexpr (CW == 4) {  // the table in LDS: R's lookups are the longest wait of a producer
+            float *lt = reinterpret_cast<float *>(lds + sizeof(BfTile<NP, CW>));
+            for (int i = threadIdx.x; i < kBfTab / 16; i += 512) ((v4f *)lt)[i] = ((const v4f *)ctab)[i];
             __syncthreads();
+            if (wave >= 4) return bf_producer<NP, CW>(T, J, lt, tile, cw, ntmax);
+        } else {
+            if (wave >= 4) return bf_producer<NP, CW>(T, J, ctab, tile, cw, ntmax);
         }
-    }
-#pragma unroll
-    for (int j = 0; j < NCW; ++j) {
-        const int f = fb + (cl0 + j) * 16 + lc;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int64_t k = k0 + pw + 4 * lr + r;
-            if (f < nF && k < M) gstore(V + (int64_t)f * ldv + k, sum[j][r]);
+        const int c0 = tb * cw / CW, nt = tb * (cw + 1) / CW - c0;
+        const char *zero = (const char *)(tab + kBoysTableDoubles) + (threadIdx.x & 63) * 16;
+        if constexpr (NTHI >= 3) {
+            if (nt == 3) return bf_consumer<NP, CW, 3>(lds, T, J, zero, tile, wave, tb0 + c0, ntmax);
         }
-    }
+        if constexpr (NTLO <= 2 && NTHI >= 2) {
+            if (nt == 2) return bf_consumer<NP, CW, 2>(lds, T, J, zero, tile, wave, tb0 + c0, ntmax);
+        }
+        if constexpr (NTLO <= 1) {
+            if (nt == 1) return bf_consumer<NP, CW, 1>(lds, T, J, zero, tile, wave, tb0 + c0, ntmax);
+        }
     }
 }
 
-template <int NP, int NFB>
-__global__ void __launch_bounds__(kCoulThreads) k_coulomb_ws_bf16(CoulJob<__bf16> J, const double *__restrict__ tab) {
-    __shared__ Bf16TileLds<NP, NFB> lds;
-    coulomb_tile_bf16<NP, NFB>(lds, J.chunks, J.nchunks, J.nsteps, J.pP, (const __bf16 *)J.H, J.nct, J.X, J.Y, J.Z, J.M,
-                               J.nF, J.V, J.ldv, tab, blockIdx.x, blockIdx.y, J.far, J.farw);
+__host__ __device__ inline int bf_col_waves(int nct, int ncb) {
+    const int tb = (nct + ncb - 1) / ncb;
+    return tb <= 3 ? 1 : tb <= 6 ? 2 : 4;
+}
+int64_t bf16_items(int64_t M, int nct, int ncb) {
+    const int64_t tiles = (M + 63) / 64;
+    return bf_col_waves(nct, ncb) == 4 ? tiles : (tiles + 1) / 2;
+}
+
+template <int NP, int CW, int NTM>
+__global__ void __launch_bounds__(512, 2) k_coulomb_bf16(CoulJob<__bf16> J, const double *__restrict__ tab) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bf_lds<NP, CW>];
+    coulomb_tile_bf16<NP, CW, (NTM > 1 ? NTM - 1 : 1), NTM>(lds, J, tab, blockIdx.x, blockIdx.y);
 }
 
 template <int NP>
-constexpr size_t bf16_lds_bytes() {
-    size_t b = sizeof(Bf16TileLds<NP, 64>);
-    b = b > sizeof(Bf16TileLds<NP, 128>) ? b : sizeof(Bf16TileLds<NP, 128>);
-    b = b > sizeof(Bf16TileLds<NP, 192>) ? b : sizeof(Bf16TileLds<NP, 192>);
-    return b;
-}
-template <int NP>
-__global__ void __launch_bounds__(kCoulThreads) k_coulomb_ws_bf16_batch_all(const CoulJob<__bf16> *__restrict__ jobs,
-                                                                            const int64_t *__restrict__ off,
-                                                                            int njobs, const double *__restrict__ tab) {
-    __shared__ __attribute__((aligned(16))) unsigned char raw[bf16_lds_bytes<NP>()];
+__global__ void __launch_bounds__(512, 2) k_coulomb_bf16_batch_all(const CoulJob<__bf16> *__restrict__ jobs,
+                                                                   const int64_t *__restrict__ off, int njobs,
+                                                                   const double *__restrict__ tab) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bf_lds_all<NP>];
     int64_t local = 0;
     const int j = job_of_block(off, njobs, (int64_t)blockIdx.x, local);
     const CoulJob<__bf16> J = uniform_job(jobs, j);
-    const int64_t tile = local / J.ncb;
-    const int cb = (int)(local - tile * J.ncb);
-#define FLOSIC_TILE_BF(NFB)                                                                                         \
-    coulomb_tile_bf16<NP, NFB>(*reinterpret_cast<Bf16TileLds<NP, NFB> *>(raw), J.chunks, J.nchunks, J.nsteps, J.pP, \
-                               (const __bf16 *)J.H, J.nct, J.X, J.Y, J.Z, J.M, J.nF, J.V, J.ldv, tab, tile, cb,  \
-                               J.far, J.farw)
-    switch (J.nfb) {
-        case 64: FLOSIC_TILE_BF(64); break;
-        case 128: FLOSIC_TILE_BF(128); break;
-        default: FLOSIC_TILE_BF(192); break;
+    const int64_t item = local / J.ncb;
+    const int cb = (int)(local - item * J.ncb);
+    switch (bf_col_waves(J.nct, J.ncb)) {
+        case 1: coulomb_tile_bf16<NP, 1, 1, 3>(lds, J, tab, item, cb); break;
+        case 2: coulomb_tile_bf16<NP, 2, 2, 3>(lds, J, tab, item, cb); break;
+        default: coulomb_tile_bf16<NP, 4, 1, 3>(lds, J, tab, item, cb); break;
     }
-#undef FLOSIC_TILE_BF
 }
 
 void launch_split_h(int npieces, const ChunkDev *chunks, int nchunks, const double *H, int ldh, int nF,
@@ -480,40 +651,37 @@ void launch_split_h(int npieces, const ChunkDev *chunks, int nchunks, const doub
         hipLaunchKernelGGL((k_split_h<3>), dim3(nchunks), dim3(256), 0, s, chunks, H, ldh, nF, nsteps, Hs);
 }
 
-void launch_coulomb_bf16(int npieces, const ChunkDev *chunks, int nchunks, int64_t nsteps, const double4 *pairP,
-                         const __bf16 *Hs, int ldh, const double *x, const double *y, const double *z, int64_t M,
-                         const double *btab, int nF, double *V, int64_t ldv, hipStream_t s, int nfb,
-                         const unsigned *far, int farw) {
-    if (nchunks <= 0 || M <= 0) return;
-    if (nfb <= 0) nfb = coulomb_cols_split(nF);
-    const CoulJob<__bf16> J{chunks, nchunks, pairP, Hs, ldh / 16, x, y, z, M, nF, V, ldv, nsteps, ldh / nfb, nfb,
-                            npieces == 3 ? far : nullptr, npieces == 3 ? farw : 0, FpSegs{}};
-    const dim3 grid((unsigned)((M + 63) / 64), (unsigned)(ldh / nfb)), blk(kCoulThreads);
-#define FLOSIC_WSB(NP, NFB) hipLaunchKernelGGL((k_coulomb_ws_bf16<NP, NFB>), grid, blk, 0, s, J, btab)
-#define FLOSIC_WSB_NFB(NP)                        \
-    switch (nfb) {                                \
-        case 64: FLOSIC_WSB(NP, 64); break;       \
-        case 128: FLOSIC_WSB(NP, 128); break;     \
-        default: FLOSIC_WSB(NP, 192); break;      \
+void launch_coulomb_bf16(int npieces, const CoulJob<__bf16> &J, const double *btab, hipStream_t s) {
+    if (J.nchunks <= 0 || J.M <= 0) return;
+    const int cw = bf_col_waves(J.nct, J.ncb), tb = (J.nct + J.ncb - 1) / J.ncb, ntm = (tb + cw - 1) / cw;
+    const dim3 grid((unsigned)bf16_items(J.M, J.nct, J.ncb), (unsigned)J.ncb), blk(512);
+#define FLOSIC_BFL(NP, CW, NTM) hipLaunchKernelGGL((k_coulomb_bf16<NP, CW, NTM>), grid, blk, 0, s, J, btab)
+#define FLOSIC_BFN(NP)                           \
+    switch (10 * cw + ntm) {                     \
+        case 11: FLOSIC_BFL(NP, 1, 1); break;    \
+        case 12: FLOSIC_BFL(NP, 1, 2); break;    \
+        case 13: FLOSIC_BFL(NP, 1, 3); break;    \
+        case 22: FLOSIC_BFL(NP, 2, 2); break;    \
+        case 23: FLOSIC_BFL(NP, 2, 3); break;    \
+        case 42: FLOSIC_BFL(NP, 4, 2); break;    \
+        default: FLOSIC_BFL(NP, 4, 3); break;    \
     }
     if (npieces == 2) {
-        FLOSIC_WSB_NFB(2)
+        FLOSIC_BFN(2)
     } else {
-        FLOSIC_WSB_NFB(3)
+        FLOSIC_BFN(3)
     }
-#undef FLOSIC_WSB_NFB
-#undef FLOSIC_WSB
+#undef FLOSIC_BFN
+#undef FLOSIC_BFL
 }
 
 void launch_coulomb_bf16_batch_all(int npieces, const CoulJob<__bf16> *jobs, const int64_t *off, int njobs,
                                    int64_t items, const double *btab, hipStream_t s) {
     if (njobs <= 0 || items <= 0) return;
     if (npieces == 2)
-        hipLaunchKernelGGL((k_coulomb_ws_bf16_batch_all<2>), dim3((unsigned)items), dim3(kCoulThreads), 0, s, jobs, off,
-                           njobs, btab);
+        hipLaunchKernelGGL((k_coulomb_bf16_batch_all<2>), dim3((unsigned)items), dim3(512), 0, s, jobs, off, njobs, btab);
     else
-        hipLaunchKernelGGL((k_coulomb_ws_bf16_batch_all<3>), dim3((unsigned)items), dim3(kCoulThreads), 0, s, jobs, off,
-                           njobs, btab);
+        hipLaunchKernelGGL((k_coulomb_bf16_batch_all<3>), dim3((unsigned)items), dim3(512), 0, s, jobs, off, njobs, btab);
 }
 
 }  // namespace flosic

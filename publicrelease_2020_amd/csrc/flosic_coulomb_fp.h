@@ -90,16 +90,6 @@ struct FpTileLds {
     __attribute__((aligned(16))) unsigned char raw[4][kWave];
 };
 
-__device__ __forceinline__ void wave_lds_sync() {  // this wave's LDS stores before its later loads (no instruction)
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-template <int CW>
-__device__ __forceinline__ void tile_sync() {  // the waves that share R
-    if constexpr (CW == 1) wave_lds_sync();
-    else __syncthreads();
-}
-
 template <typename T, int NT>
 struct FpAcc {
     typename MfmaTraits<T>::acc a[4][NT];
@@ -355,7 +345,7 @@ void launch_coulomb_mfma(const FpSegs &seg, const double4 *pairP, const T *Hf, c
     J.nF = nF;
     J.V = V;
     J.ldv = ldv;
-    J.ncb = fp_col_blocks(nF, nfb);
+    J.ncb = coulomb_col_blocks(nF, nfb);
     const int cw = fp_col_waves(J.nct, J.ncb), tb = (J.nct + J.ncb - 1) / J.ncb, ntm = (tb + cw - 1) / cw;
     const dim3 grid((unsigned)((M + 63) / 64), (unsigned)J.ncb), blk(256);
 #define FLOSIC_FP(CW, NTM) hipLaunchKernelGGL((k_coulomb_fp<T, CW, NTM>), grid, blk, 0, s, J, btab)

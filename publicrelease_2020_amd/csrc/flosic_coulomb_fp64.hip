@@ -4,7 +4,7 @@
 namespace flosic {
 
 int64_t fp_steps(const FpSegs &seg) { return seg_step0(seg, 5); }
-int fp_col_blocks(int nF, int nfb) {
+int coulomb_col_blocks(int nF, int nfb) {
     const int tb = std::min(nfb / 16, 12);  // column tiles of a block
     return std::max(1, ((nF + 15) / 16 + tb - 1) / tb);
 }

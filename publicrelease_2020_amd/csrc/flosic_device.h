@@ -62,55 +62,75 @@ __host__ __device__ constexpr int tuv_comp(int i, int which) {
 // Boys F_0..F_TOP of the reference scheme (fffmt3.F): T > 16 one-term asymptote and upward recursion, else the
 // cubic Taylor expansion of F_TOP about the nearest table node and downward recursion.  C = double for the FP64
 // forms; C = float (table rounded to FP32) where R feeds FP32 or split-BF16 MFMA operands anyway.
+// The FP32 branches, with their rounding steps written out (see rterm): far (T > 16) and near, the hardware reciprocal and
+// square root (1 ulp) instead of correctly rounded ones, well inside the FP32 R's own rounding
+template <int TOP>
+__device__ __forceinline__ void boys32_far(float T, float eT, float *F) {
+    const float rect1 = 0.5f * __builtin_amdgcn_rcpf(T);
+    const float q = __builtin_fmaf(__builtin_amdgcn_sqrtf(T), 1.77245385090551602728f, -eT);
+    F[0] = rect1 * q;
+    F[1] = rect1 * __builtin_fmaf(rect1, q, -eT);
+#pragma unroll
+    for (int m = 2; m <= TOP; ++m) F[m] = rect1 * __builtin_fmaf((float)(2 * m - 1), F[m - 1], -eT);
+}
+template <int TOP>
+__device__ __forceinline__ void boys32_near(float T, float eT, const float *__restrict__ tab, float *F) {
+    const int it = (int)__builtin_fmaf(100.0f, T, 1.5f);
+    const float dt = __builtin_fmaf(1.0e-2f, (float)(it - 1), -T);
+    const float *f = tab + (it - 1) * kBoysCols;
+    // times the rounded 1/6 (a correctly rounded division costs 10 VALU)
+    F[TOP] = __builtin_fmaf(dt, __builtin_fmaf(dt, __builtin_fmaf(f[TOP + 2], 0.5f, dt * (f[TOP + 3] * (1.0f / 6.0f))), f[TOP + 1]),
+                            f[TOP]);
+    const float rect1 = 2.0f * T;
+#pragma unroll
+    for (int m = TOP - 1; m >= 0; --m) {
+        const float r = __builtin_fmaf(rect1, F[m + 1], eT);
+        F[m] = m == 0 ? r : r * (1.0f / (2 * m + 1));
+    }
+}
 template <int TOP, typename C>
 __device__ __forceinline__ void boys(C T, C eT, const C *__restrict__ tab, C *F) {
-    if (T > C(16.0)) {
-        // FP32: the hardware reciprocal and square root (1 ulp) instead of correctly rounded ones, well inside the
-        // FP32 R's own rounding; FP64 keeps the reference scheme's operations
-        C rect1, rt;
-        if constexpr (sizeof(C) == 4) {
-            rect1 = 0.5f * __builtin_amdgcn_rcpf(T);
-            rt = __builtin_amdgcn_sqrtf(T);
-        } else {
-            rect1 = C(0.5) / T;
-            rt = sqrt(T);
-        }
-        F[0] = rect1 * (rt * C(1.77245385090551602728) - eT);
+    if constexpr (sizeof(C) == 4) {
+        if (T > 16.0f) boys32_far<TOP>(T, eT, F);
+        else boys32_near<TOP>(T, eT, tab, F);
+    } else if (T > 16.0) {
+        const double rect1 = 0.5 / T, rt = sqrt(T);
+        F[0] = rect1 * (rt * 1.77245385090551602728 - eT);
 #pragma unroll
         for (int m = 1; m <= TOP; ++m) F[m] = rect1 * ((2 * m - 1) * F[m - 1] - eT);
     } else {
-        const int it = (int)(C(100.0) * T + C(1.5));
-        const C dt = C(1.0e-2) * (it - 1) - T;
-        const C *f = tab + (it - 1) * kBoysCols;
-        if constexpr (sizeof(C) == 4)  // FP32: times the rounded 1/6 (a correctly rounded division costs 10 VALU)
-            F[TOP] = f[TOP] + dt * (f[TOP + 1] + dt * (f[TOP + 2] * 0.5f + dt * (f[TOP + 3] * (1.0f / 6.0f))));
-        else
-            F[TOP] = f[TOP] + dt * (f[TOP + 1] + dt * (f[TOP + 2] / C(2.0) + dt * (f[TOP + 3] / C(6.0))));
-        const C rect1 = C(2.0) * T;
+        const int it = (int)(100.0 * T + 1.5);
+        const double dt = 1.0e-2 * (it - 1) - T;
+        const double *f = tab + (it - 1) * kBoysCols;
+        F[TOP] = f[TOP] + dt * (f[TOP + 1] + dt * (f[TOP + 2] / 2.0 + dt * (f[TOP + 3] / 6.0)));
+        const double rect1 = 2.0 * T;
 #pragma unroll
         for (int m = TOP - 1; m >= 0; --m) {
-            const C r = F[m + 1] * rect1 + eT;
-            F[m] = (m == 0) ? r : r * (C(1.0) / (2 * m + 1));
+            const double r = F[m + 1] * rect1 + eT;
+            F[m] = (m == 0) ? r : r * (1.0 / (2 * m + 1));
         }
     }
 }
 
+// x r0 + c r1.  FP32: with the rounding steps written out, so that every kernel that generates R in FP32 gets the same bits
+template <int c, typename C>
+__device__ __forceinline__ C rterm(C x, C r0, C r1) {
+    if constexpr (sizeof(C) == 4) return c == 1 ? __builtin_fmaf(x, r0, r1) : __builtin_fmaf((float)c, r1, x * r0);
+    else return x * r0 + c * r1;
+}
 // one Hermite step R^{(n)}_I from R^{(n+1)} in place (entries of lower order still hold level n+1)
 template <int I, typename C>
 __device__ __forceinline__ void rstep(C *R, C X, C Y, C Z) {
     constexpr int t = tuv_comp(I, 0), u = tuv_comp(I, 1), v = tuv_comp(I, 2);
     if constexpr (t > 0) {
-        C r = X * R[tuv_idx(t - 1, u, v)];
-        if constexpr (t > 1) r += (t - 1) * R[tuv_idx(t - 2, u, v)];
-        R[I] = r;
+        if constexpr (t > 1) R[I] = rterm<t - 1, C>(X, R[tuv_idx(t - 1, u, v)], R[tuv_idx(t - 2, u, v)]);
+        else R[I] = X * R[tuv_idx(t - 1, u, v)];
     } else if constexpr (u > 0) {
-        C r = Y * R[tuv_idx(t, u - 1, v)];
-        if constexpr (u > 1) r += (u - 1) * R[tuv_idx(t, u - 2, v)];
-        R[I] = r;
+        if constexpr (u > 1) R[I] = rterm<u - 1, C>(Y, R[tuv_idx(t, u - 1, v)], R[tuv_idx(t, u - 2, v)]);
+        else R[I] = Y * R[tuv_idx(t, u - 1, v)];
     } else {
-        C r = Z * R[tuv_idx(t, u, v - 1)];
-        if constexpr (v > 1) r += (v - 1) * R[tuv_idx(t, u, v - 2)];
-        R[I] = r;
+        if constexpr (v > 1) R[I] = rterm<v - 1, C>(Z, R[tuv_idx(t, u, v - 1)], R[tuv_idx(t, u, v - 2)]);
+        else R[I] = Z * R[tuv_idx(t, u, v - 1)];
     }
 }
 template <int I, typename C>
@@ -133,7 +153,9 @@ __device__ __forceinline__ void rlevels(C *R, C X, C Y, C Z, const C *F, const C
 template <int L, typename C = double>
 __device__ __forceinline__ void hermite_R(C p, C X, C Y, C Z, const C *__restrict__ tab, C *R) {
     constexpr int TOP = L < 2 ? 2 : L;
-    const C T = p * (X * X + Y * Y + Z * Z);
+    C T;
+    if constexpr (sizeof(C) == 4) T = p * __builtin_fmaf(Z, Z, __builtin_fmaf(X, X, Y * Y));
+    else T = p * (X * X + Y * Y + Z * Z);
     C F[TOP + 1];
     C eT;
     if constexpr (sizeof(C) == 8)
@@ -188,6 +210,18 @@ __device__ __forceinline__ ChunkDev chunk_at(const ChunkDev *__restrict__ chunks
     __builtin_memcpy(&ch, w, sizeof(ch));
     return ch;
 }
+// s_waitcnt lgkmcnt(0) alone (vmcnt 63, expcnt 7)
+__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xF | (7 << 4) | (0 << 8) | (3 << 14)); }
+__device__ __forceinline__ void wave_lds_sync() {  // this wave's LDS stores before its later loads (no instruction)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <int CW>
+__device__ __forceinline__ void tile_sync() {  // the waves that share R
+    if constexpr (CW == 1) wave_lds_sync();
+    else __syncthreads();
+}
+
 // the type in which R is generated: FP64 for the FP64 form, FP32 for the FP32 and split-BF16 operands
 template <typename T>
 using RType = typename std::conditional<sizeof(T) == 8, double, float>::type;

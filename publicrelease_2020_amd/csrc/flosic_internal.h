@@ -43,12 +43,17 @@ struct PairDev {
 // chunk of consecutive groups of one order L (split-BF16 forms): Hermite rows [hrow0, hrow0 + (pe-pb)*ntuv(L)) staged
 // in LDS and zero-extended to kr rows (a multiple of the MFMA K step)
 constexpr int kChunkRowsBf16 = 64;  // split-BF16 kernel: K step 32
-constexpr int kFarWords = 1000;     // far-chunk bits per tile the split-BF16 kernel holds in LDS (32000 chunks)
+constexpr int kFarWords = 1000;     // most 32-bit words of far-chunk bits per tile (32000 chunks)
 struct ChunkDev {
     // groups [pb, pe); L: their Hermite order, or 5 / 6 for the first 32 / last 3 rows of L = 4 groups; kr: rows after zero extension; hrow0: first Hermite row of group pb
     int pb, pe, L, kr, hrow0;
     int prow0;  // first row of the chunk in the zero-extended row space of its list (split-BF16 H layout)
+    int flush;  // the FP32 accumulators go into the FP64 sums after this chunk
 };
+// split-BF16: a chunk is marked flush once at least this many Hermite rows have been accumulated (and the last one).  On
+// the K=64 workload every 64, 128, 256, 512 rows gave |dE| against FP64 of 4.9e-7, 5.3e-7, 4.4e-7 and 6.2e-7 Ha; the
+// flush is 96 VALU instructions per wave.
+constexpr int kFlushRowsBf16 = 256;
 
 // the groups by order: those of order L are [g[L], g[L + 1])
 struct FpSegs {
@@ -78,6 +83,7 @@ struct CoulJob {
     const unsigned *far;
     int farw;
     FpSegs seg;
+    int rgc[5];  // split-BF16: four runs of chunks [rgc[i], rgc[i + 1]) of about equal length that begin after a flush
 };
 
 // Column-block widths that may be asked for: nfb must divide ldh (nF rounded up to a multiple of coulomb_cols); the
@@ -88,8 +94,10 @@ bool coulomb_cols_legal(int nfb, int ldh, bool split);
 int coulomb_cols(int nF);
 
 // per-phase launch helpers (stream-ordered)
-// host: fills kBoysRows x kBoysCols doubles followed by the same table in FP32 (kBoysTableDoubles in all)
+// host: fills kBoysRows x kBoysCols doubles followed by the same table in FP32 (kBoysTableDoubles in all); in device memory
+// kZeroDoubles zeros follow (the third H piece of far chunks, three column tiles of 1 KiB)
 constexpr int kBoysTableDoubles = kBoysRows * kBoysCols * 3 / 2;
+constexpr int kZeroDoubles = 384;
 void boys_table(double *h_tab);
 
 // nd = 1 (values), 4 (+ gradient), 10 (+ Hessian xx,yy,zz,xy,xz,yz) planes, -1 (one Laplacian plane) or -3 (the
@@ -119,7 +127,7 @@ void launch_coulomb(const int *segL /*6 offsets*/, const double4 *pairP, const i
 // kernels then generate R_tuv of every (point, group) and stream H.  T = double (FP64 MFMA) or float (FP32 MFMA, FP64
 // sums per chunk of <= 64 rows): fp_steps K steps of 4 rows, at most nfb FLO columns per block.
 int64_t fp_steps(const FpSegs &seg);
-int fp_col_blocks(int nF, int nfb);
+int coulomb_col_blocks(int nF, int nfb);
 template <typename T>
 void launch_frag_h(const FpSegs &seg, const double *H, int ldh, int nF, T *Hf, hipStream_t s);
 template <typename T>
@@ -138,14 +146,13 @@ void launch_coulomb_bf16_batch_all(int npieces, const CoulJob<__bf16> *jobs, con
 int coulomb_cols_split(int nF);
 
 // split-BF16 form: R and H split into NP = 2 or 3 bf16 pieces, 3 or 6 cross products per 16x16x32 MFMA step,
-// FP32 accumulation inside a chunk, FP64 sums across chunks.  H is split once per evaluation into
+// FP32 accumulation from flush to flush, FP64 sums.  H is split once per evaluation into
 // Hs[piece][nsteps][ldh/16][64 lanes][8].
 void launch_split_h(int npieces, const ChunkDev *chunks, int nchunks, const double *H, int ldh, int nF,
                     int64_t nsteps, __bf16 *Hs, hipStream_t s);
-void launch_coulomb_bf16(int npieces, const ChunkDev *chunks, int nchunks, int64_t nsteps, const double4 *pairP,
-                         const __bf16 *Hs, int ldh, const double *x, const double *y, const double *z, int64_t M,
-                         const double *btab, int nF, double *V, int64_t ldv, hipStream_t s, int nfb = 0,
-                         const unsigned *far = nullptr, int farw = 0);
+void launch_coulomb_bf16(int npieces, const CoulJob<__bf16> &J, const double *btab, hipStream_t s);
+// work items of a system per column block (64-point tiles, or pairs of them)
+int64_t bf16_items(int64_t M, int nct, int ncb);
 // Far-chunk bits for the three-piece split-BF16 form: bit c of word far[t * farw + c / 32] is set when every (point,
 // group) pair of 64-point tile t and chunk c of the split-BF16 chunk list has T = p|r - P|^2 > tfar (a lower bound
 // from the tile's centroid and radius); farrows[0] (zeroed here) accumulates the rows of the far (tile, chunk) pairs
