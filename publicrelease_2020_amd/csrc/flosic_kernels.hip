@@ -180,79 +180,103 @@ void launch_prim_coef(int nps, const int *ps_f0, const int *ps_stride, const int
 // ---------------------------------------------------------------------------------------------------
 // Hermite coefficients of every pair for every FLO.  E^{ij}_t along one axis by the McMurchie-Davidson
 // recursion; H[row+tuv][f] = sym * 2pi/p * sum_{mu,nu} dA[mu][f] dB[nu][f] Ex Ey Ez
+//
+// Bound: latency, a few microseconds of work per block at any system size.  One block per group: 27 threads raise the
+// E^{ij}_t of one axis and (i, j) in registers; the products Ex Ey Ez of every (component pair, tuv) go to LDS, wave = pair,
+// lane = tuv; then a thread holds one (tuv, FLO) and runs over the component pairs, up to 100, from LDS.  A thread that held all
+// 35 sums of one FLO (indexed at run time, so in scratch memory) left 54 of 64 lanes idle at 10 FLOs and took 190 us
+// there (289 groups), 229 at 30 FLOs (1686 groups), 525 at 96 FLOs (15750); now 27, 82 and 279.
 // ---------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(128) k_hermite(const PairDev *__restrict__ pairs, const double *__restrict__ dps,
-                                                  int nF, double *__restrict__ H, int ldh) {
-    __shared__ double E[3][3][3][5];
+constexpr int kHermThreads = 256, kHermCols = 64;
+__device__ __forceinline__ void e_raise(double (&v)[5], double shift, double inv2p) {
+    double o[5];
+#pragma unroll
+    for (int t = 0; t < 5; ++t) o[t] = v[t];
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+        double x = t >= 1 ? inv2p * o[t >= 1 ? t - 1 : 0] : 0.0;
+        x += shift * o[t];
+        if (t < 4) x += (t + 1) * o[t < 4 ? t + 1 : 4];
+        v[t] = x;
+    }
+}
+__global__ void __launch_bounds__(kHermThreads) k_hermite(const PairDev *__restrict__ pairs,
+                                                          const double *__restrict__ dps, int nF,
+                                                          double *__restrict__ H, int ldh) {
+    __shared__ double E[3][3][3][5], C[100 * 35], dA[10][kHermCols], dB[10][kHermCols];
     const PairDev pr = pairs[blockIdx.x];
     const double p = pr.a + pr.b;
-    if (threadIdx.x < 3) {
-        const int d = threadIdx.x;
-        const double P = (pr.a * pr.A[d] + pr.b * pr.B[d]) / p;
-        const double xpa = P - pr.A[d], xpb = P - pr.B[d];
-        const double dd = pr.A[d] - pr.B[d];
-        const double K = exp(-pr.a * pr.b / p * dd * dd);
-        const double inv2p = 0.5 / p;
-        for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j)
-                for (int t = 0; t < 5; ++t) E[d][i][j][t] = 0.0;
-        E[d][0][0][0] = K;
-        for (int i = 0; i <= 2; ++i)
-            for (int j = 0; j <= 2; ++j) {
-                if (i == 0 && j == 0) continue;
-                const int pi = i > 0 ? i - 1 : i, pj = i > 0 ? j : j - 1;
-                const double shift = i > 0 ? xpa : xpb;
-                const int np = i + j - 1;
-                for (int t = 0; t <= i + j; ++t) {
-                    double v = 0.0;
-                    if (t >= 1 && t - 1 <= np) v += inv2p * E[d][pi][pj][t - 1];
-                    if (t <= np) v += shift * E[d][pi][pj][t];
-                    if (t + 1 <= np) v += (t + 1) * E[d][pi][pj][t + 1];
-                    E[d][i][j][t] = v;
-                }
-            }
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid < 27) {
+        const int d = tid / 9, i = tid / 3 % 3, j = tid % 3;
+        const double A = d == 0 ? pr.A[0] : d == 1 ? pr.A[1] : pr.A[2], B = d == 0 ? pr.B[0] : d == 1 ? pr.B[1] : pr.B[2];
+        const double P = (pr.a * A + pr.b * B) / p;
+        const double xpa = P - A, xpb = P - B, dd = A - B, inv2p = 0.5 / p;
+        double v[5] = {exp(-pr.a * pr.b / p * dd * dd), 0.0, 0.0, 0.0, 0.0};
+        for (int q = 0; q < j; ++q) e_raise(v, xpb, inv2p);
+        for (int q = 0; q < i; ++q) e_raise(v, xpa, inv2p);
+#pragma unroll
+        for (int t = 0; t < 5; ++t) E[d][i][j][t] = v[t];
     }
-    __syncthreads();
-    const int L = pr.lA + pr.lB;
-    const int nt = ntuv(L);
+    // components of either centre: those of the shells l that it has, as bits of the component index 0..9
+    int mA = 0, mB = 0;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        const int bits = ((1 << ncart(l)) - 1) << loff(l);
+        if (l <= pr.lA && pr.psA[l] >= 0) mA |= bits;
+        if (l <= pr.lB && pr.psB[l] >= 0) mB |= bits;
+    }
+    const int nB = __builtin_popcount(mB), nA = __builtin_popcount(mA), nt = ntuv(pr.lA + pr.lB);
     const double fac = pr.sym * 2.0 * M_PI / p;
-    for (int f = threadIdx.x; f < ldh; f += blockDim.x) {
-        if (f >= nF) {
-            for (int t = 0; t < nt; ++t) H[(int64_t)(pr.row + t) * ldh + f] = 0.0;
-            continue;
-        }
-        double h[35];
-        for (int t = 0; t < 35; ++t) h[t] = 0.0;
-        for (int la = 0; la <= pr.lA; ++la) {
-            if (pr.psA[la] < 0) continue;
-            for (int m = 0; m < ncart(la); ++m) {
-                const double da = dps[((int64_t)pr.psA[la] * 6 + m) * nF + f];
-                if (da == 0.0) continue;
-                const int ax = cpow(loff(la) + m, 0), ay = cpow(loff(la) + m, 1), az = cpow(loff(la) + m, 2);
-                for (int lb = 0; lb <= pr.lB; ++lb) {
-                    if (pr.psB[lb] < 0) continue;
-                    for (int n = 0; n < ncart(lb); ++n) {
-                        const double dab = da * dps[((int64_t)pr.psB[lb] * 6 + n) * nF + f];
-                        if (dab == 0.0) continue;
-                        const int bx = cpow(loff(lb) + n, 0), by = cpow(loff(lb) + n, 1), bz = cpow(loff(lb) + n, 2);
-                        for (int t = 0; t <= ax + bx; ++t) {
-                            const double et = dab * E[0][ax][bx][t];
-                            for (int u = 0; u <= ay + by; ++u) {
-                                const double etu = et * E[1][ay][by][u];
-                                for (int v = 0; v <= az + bz; ++v) h[tuv_idx(t, u, v)] += etu * E[2][az][bz][v];
-                            }
-                        }
-                    }
-                }
+    __syncthreads();
+    {
+        // (t, u, v) of entry `lane`: order, then the position in its block: t falls by one after 1, 2, 3, .. entries
+        const int ord = lane < 1 ? 0 : lane < 4 ? 1 : lane < 10 ? 2 : lane < 20 ? 3 : 4;
+        const int pos = min(lane, 34) - ord * (ord + 1) * (ord + 2) / 6;
+        const int uv = pos < 1 ? 0 : pos < 3 ? 1 : pos < 6 ? 2 : pos < 10 ? 3 : 4;
+        const int t = ord - uv, v = pos - uv * (uv + 1) / 2, u = uv - v;
+        int e = 0;
+        for (int ma = mA; ma; ma &= ma - 1) {
+            const int a = __builtin_ctz(ma), ax = cpow(a, 0), ay = cpow(a, 1), az = cpow(a, 2);
+            for (int mb = mB; mb; mb &= mb - 1, ++e) {
+                if ((e & 3) != wave) continue;
+                const int b = __builtin_ctz(mb), bx = cpow(b, 0), by = cpow(b, 1), bz = cpow(b, 2);
+                if (lane < nt) C[e * nt + lane] = E[0][ax][bx][t] * E[1][ay][by][u] * E[2][az][bz][v];
             }
         }
-        for (int t = 0; t < nt; ++t) H[(int64_t)(pr.row + t) * ldh + f] = fac * h[t];
+    }
+    // columns at a time (of ldh, nF rounded up to 16)
+    const int sh = ldh > 32 ? 6 : ldh > 16 ? 5 : 4, cols = 1 << sh;
+    for (int f0 = 0; f0 < ldh; f0 += cols) {
+        __syncthreads();
+        for (int x = tid; x < (nA + nB) << sh; x += kHermThreads) {
+            const int f = f0 + (x & (cols - 1)), c = x >> sh;
+            const bool isA = c < nA;
+            int m = isA ? mA : mB;
+            for (int q = isA ? c : c - nA; q > 0; --q) m &= m - 1;
+            const int k = __builtin_ctz(m), l = k < loff(1) ? 0 : k < loff(2) ? 1 : 2;
+            const int ps = isA ? (l == 0 ? pr.psA[0] : l == 1 ? pr.psA[1] : pr.psA[2])
+                               : (l == 0 ? pr.psB[0] : l == 1 ? pr.psB[1] : pr.psB[2]);
+            (isA ? dA[c] : dB[c - nA])[x & (cols - 1)] = f < nF ? dps[((int64_t)ps * 6 + k - loff(l)) * nF + f] : 0.0;
+        }
+        __syncthreads();
+        for (int x = tid; x < nt << sh; x += kHermThreads) {
+            const int fl = x & (cols - 1), tuv = x >> sh;
+            if (f0 + fl >= ldh) continue;
+            const double *c = C + tuv;
+            double h = 0.0;
+            for (int m = 0; m < nA; ++m) {
+                const double da = dA[m][fl];
+                for (int n = 0; n < nB; ++n, c += nt) h += da * dB[n][fl] * *c;
+            }
+            H[(int64_t)(pr.row + tuv) * ldh + f0 + fl] = fac * h;
+        }
     }
 }
 
 void launch_hermite(int ngroup, const PairDev *pairs, const double *dps, int nF, double *H, int ldh, hipStream_t s) {
     if (ngroup <= 0) return;
-    hipLaunchKernelGGL(k_hermite, dim3(ngroup), dim3(128), 0, s, pairs, dps, nF, H, ldh);
+    hipLaunchKernelGGL(k_hermite, dim3(ngroup), dim3(kHermThreads), 0, s, pairs, dps, nF, H, ldh);
 }
 
 template <int L, int CH>
