@@ -116,6 +116,29 @@ struct DevBuf {
     }
 };
 
+// Pinned host memory of a context: copies to and from it are asynchronous and cost the host a few microseconds, where a
+// copy from or to ordinary memory waits for the stream and costs 15 to 30
+struct PinBuf {
+    double *p = nullptr;
+    size_t n = 0;
+    ~PinBuf() {
+        if (p) (void)hipHostFree(p);
+    }
+    // at least cnt doubles; the contents are lost when it grows, and copies on s that still use it are waited for
+    bool ensure(size_t cnt, hipStream_t s) {
+        if (cnt <= n) return true;
+        if (p && (hipStreamSynchronize(s) != hipSuccess || hipHostFree(p) != hipSuccess)) return false;
+        p = nullptr;
+        n = 0;
+        if (hipHostMalloc((void **)&p, cnt * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+            p = nullptr;
+            return false;
+        }
+        n = cnt;
+        return true;
+    }
+};
+
 struct Spin {
     int nwf = 0, nocc = 0;
     std::vector<double> coef;  // nbas x nwf col-major
@@ -131,8 +154,6 @@ struct Spin {
     std::vector<double> vab;      // n^3
     std::vector<double> debdax, grad;  // 3 x n
     DevBuf<double> d_ctil;        // nbas x nwf: FLOs then virtual KS orbitals
-    DevBuf<double> d_cocc;        // nbas x nocc: occupied KS orbitals
-    DevBuf<double> d_psi, d_tmat;  // orbitals at the FODs (4 x n x n), TMAT
 };
 
 }  // namespace
@@ -204,9 +225,12 @@ struct flosic_ctx {
     // evaluation buffers
     int nF = 0, ldh = 0;  // ldh: nF rounded up to the widest column block (the legal block widths divide it)
     int ldc = 0;          // leading dimension of H: nF rounded up to 16
-    DevBuf<double> d_fodxyz, d_fodchi;  // FOD coordinates of both spins (x, y, z arrays), basis planes at them
-    DevBuf<double> d_cflo, d_dps, d_H, d_phi, d_VH, d_Vtot, d_U, d_part, d_energy, d_G, d_Gpart, d_vabpart, d_vab,
-        d_lambda, d_asy, d_Ux, d_lamex, d_dft, d_dftpart, d_dplanes, d_dphi, d_dvt, d_du, d_dG;
+    // Fermi-orbital stage, both spins: FOD coordinates (x, y, z arrays) and KS orbitals (FoLayout); basis planes, orbitals
+    // at the FODs (4 x n x n each); TMAT
+    DevBuf<double> d_foin, d_fodchi, d_psi, d_tmat;
+    PinBuf h_fo, h_res, h_pot;  // host side of d_foin, d_psi and d_tmat, of d_res, of d_pot
+    DevBuf<double> d_cflo, d_dps, d_H, d_phi, d_VH, d_Vtot, d_U, d_part, d_G, d_Gpart, d_vabpart, d_vab,
+        d_res /* results for the host: ResLayout */, d_Ux, d_dft, d_dftpart, d_dplanes, d_dphi, d_dvt, d_du, d_dG;
     std::vector<double> h_energy, h_asy;
     double zsic = 0.0;
     bool evaluated = false, fo_done = false;
@@ -447,7 +471,7 @@ void eigh_sym(int n, const double *Ain, double *q, double *U) {
 // FMAT, OVER, the Lowdin eigen-decomposition, S^-1/2 and TMAT of one spin on the host (frmorb2.F:140-290,
 // lowden_files.F) from Psi_K(j, i) = d_K psi_j at FOD i (K = 0 value, 1..3 gradient; psiK[K][i][j]); returns 0, or
 // the 1-based index of a Lowdin eigenvalue below 1e-8
-int lowdin_host(Spin &s, const std::vector<double> &psiK) {
+int lowdin_host(Spin &s, const double *psiK) {
     const int n = s.nocc;
     const size_t nn = (size_t)n * n;
     s.fmat.assign(nn * 4, 0.0);
@@ -913,64 +937,78 @@ int check_ready(flosic_ctx *c) {
 // FODs of both spins as its points), Psi_K = C^T chi_K at the FODs (4 products of nocc x nbas x nocc per spin,
 // rocBLAS), the n x n Lowdin algebra of the two spins on two host threads, then cflo = C_occ TMAT^T (rocBLAS); the FLO
 // coefficients of all FLOs land in d_cflo (nbas x nF, spin 1 first)
+// offsets (doubles) in d_foin: 3 x nfod coordinates, then C (nbas x nwf) of both spins; in d_tmat: n x n of both spins
+struct FoLayout {
+    size_t coef[2], tm[2], total, ntm;
+    explicit FoLayout(const flosic_ctx *c) {
+        const size_t n0 = c->sp[0].nocc, n1 = c->sp[1].nocc;
+        coef[0] = 3 * (n0 + n1);
+        coef[1] = coef[0] + c->sp[0].coef.size();
+        total = coef[1] + c->sp[1].coef.size();
+        tm[0] = 0;
+        tm[1] = n0 * n0;
+        ntm = tm[1] + n1 * n1;
+    }
+};
 int run_frmorb(flosic_ctx *c) {
     const int N = c->nbas;
     const int n0 = c->sp[0].nocc, nfod = n0 + c->sp[1].nocc;
     ALLOC(c, c->d_cflo, (size_t)N * nfod);
-    int r = 0;
-    {   // FOD coordinates of both spins as three point arrays; chi planes [K][mu][FOD], K = value, d/dx, d/dy, d/dz
-        std::vector<double> xyz(3 * (size_t)nfod);
-        for (int t = 0; t < nfod; ++t) {
-            const double *f = t < n0 ? &c->sp[0].fod[3 * t] : &c->sp[1].fod[3 * (t - n0)];
-            for (int d = 0; d < 3; ++d) xyz[(size_t)d * nfod + t] = f[d];
-        }
-        if ((r = upload(c, c->d_fodxyz, xyz))) return r;
-        ALLOC(c, c->d_fodchi, 4 * (size_t)N * nfod);
-        launch_fill_zero(c->d_fodchi.p, 4 * (size_t)N * nfod, c->stream);
-        if (nfod > 0)
-            launch_basis_planes<double>(basis_view(c), c->d_fodxyz.p, c->d_fodxyz.p + nfod, c->d_fodxyz.p + 2 * nfod,
-                                        nfod, 4, c->d_fodchi.p, nfod, c->stream);
-        HIPCHK(c, hipGetLastError());
+    // One copy brings the FOD coordinates and the KS orbitals of both spins, one takes the orbitals at the FODs back, one
+    // brings both TMAT; the only wait is the one for the middle one.  (Eight copies out of and into ordinary memory, each
+    // waiting for the stream, made this stage 0.2 ms of host time at any size.)  The staging memory is free again when
+    // it is written: every pass waits for its own orbitals at the FODs, which lie behind the copies of the pass before.
+    const FoLayout fo(c);
+    const size_t npsi = 4 * fo.ntm;
+    ALLOC(c, c->d_foin, fo.total);
+    ALLOC(c, c->d_fodchi, 4 * (size_t)N * nfod);
+    ALLOC(c, c->d_psi, npsi);
+    ALLOC(c, c->d_tmat, fo.ntm);
+    if (!c->h_fo.ensure(fo.total + npsi + fo.ntm, c->stream)) return fail(c, FLOSIC_ENOMEM, "host staging memory");
+    double *h_in = c->h_fo.p, *h_psi = h_in + fo.total, *h_tmat = h_psi + npsi;
+    for (int t = 0; t < nfod; ++t) {
+        const double *f = t < n0 ? &c->sp[0].fod[3 * t] : &c->sp[1].fod[3 * (t - n0)];
+        for (int d = 0; d < 3; ++d) h_in[(size_t)d * nfod + t] = f[d];
     }
-    std::vector<double> psiK[2];
+    for (int s = 0; s < 2; ++s) std::copy(c->sp[s].coef.begin(), c->sp[s].coef.end(), h_in + fo.coef[s]);
+    HIPCHK(c, hipMemcpyAsync(c->d_foin.p, h_in, sizeof(double) * fo.total, hipMemcpyHostToDevice, c->stream));
+    // chi planes [K][mu][FOD], K = value, d/dx, d/dy, d/dz
+    launch_fill_zero(c->d_fodchi.p, 4 * (size_t)N * nfod, c->stream);
+    if (nfod > 0)
+        launch_basis_planes<double>(basis_view(c), c->d_foin.p, c->d_foin.p + nfod, c->d_foin.p + 2 * nfod, nfod, 4,
+                                    c->d_fodchi.p, nfod, c->stream);
+    HIPCHK(c, hipGetLastError());
+    const double one = 1.0, zero = 0.0;
     for (int s = 0, off = 0; s < 2; off += c->sp[s].nocc, ++s) {
-        Spin &sp = c->sp[s];
-        const int n = sp.nocc;
+        const int n = c->sp[s].nocc;
         if (n == 0) continue;
         const size_t nn = (size_t)n * n;
-        if ((r = upload(c, sp.d_cocc, sp.coef.data(), (size_t)N * n))) return r;
-        ALLOC(c, sp.d_psi, 4 * nn);
         // Psi_K(j, i) = sum_mu C(mu, j) chi_K(mu, a_i): C^T times the transpose of the [mu][FOD] plane of this spin's FODs
-        const double one = 1.0, zero = 0.0;
         BLASCHK(c, rocblas_dgemm_strided_batched(c->blas, rocblas_operation_transpose, rocblas_operation_transpose, n, n,
-                                                 N, &one, sp.d_cocc.p, N, 0, c->d_fodchi.p + off, nfod,
-                                                 (rocblas_stride)N * nfod, &zero, sp.d_psi.p, n, (rocblas_stride)nn, 4));
-        psiK[s].resize(4 * nn);
-        HIPCHK(c, hipMemcpyAsync(psiK[s].data(), sp.d_psi.p, sizeof(double) * 4 * nn, hipMemcpyDeviceToHost,
-                                 c->stream));
+                                                 N, &one, c->d_foin.p + fo.coef[s], N, 0, c->d_fodchi.p + off, nfod,
+                                                 (rocblas_stride)N * nfod, &zero, c->d_psi.p + 4 * fo.tm[s], n,
+                                                 (rocblas_stride)nn, 4));
     }
+    HIPCHK(c, hipMemcpyAsync(h_psi, c->d_psi.p, sizeof(double) * npsi, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     int bad[2] = {0, 0};
     host_parallel(2, [&](int s0, int s1) {
         for (int s = s0; s < s1; ++s)
-            if (c->sp[s].nocc > 0) bad[s] = lowdin_host(c->sp[s], psiK[s]);
+            if (c->sp[s].nocc > 0) bad[s] = lowdin_host(c->sp[s], h_psi + 4 * fo.tm[s]);
     }, std::min(n0, nfod - n0) >= kThreadMinOrbitals);
     for (int s = 0; s < 2; ++s)
         if (bad[s])
             return fail(c, FLOSIC_ELOWDIN, "Lowdin eigenvalue %d = %.3e < 1e-8 (coincident FODs?)", bad[s],
                         c->sp[s].q[bad[s] - 1]);
-    int off = 0;
-    for (int s = 0; s < 2; ++s) {
-        Spin &sp = c->sp[s];
-        const int n = sp.nocc;
-        if (n > 0) {
-            if ((r = upload(c, sp.d_tmat, sp.tmat))) return r;
-            // cflo(mu, i) = sum_j C(mu, j) TMAT(i, j)
-            const double one = 1.0, zero = 0.0;
+    for (int s = 0; s < 2; ++s)
+        if (c->sp[s].nocc > 0) std::copy(c->sp[s].tmat.begin(), c->sp[s].tmat.end(), h_tmat + fo.tm[s]);
+    HIPCHK(c, hipMemcpyAsync(c->d_tmat.p, h_tmat, sizeof(double) * fo.ntm, hipMemcpyHostToDevice, c->stream));
+    for (int s = 0, off = 0; s < 2; off += c->sp[s].nocc, ++s) {
+        const int n = c->sp[s].nocc;
+        if (n > 0)  // cflo(mu, i) = sum_j C(mu, j) TMAT(i, j)
             BLASCHK(c, rocblas_dgemm(c->blas, rocblas_operation_none, rocblas_operation_transpose, N, n, n, &one,
-                                     sp.d_cocc.p, N, sp.d_tmat.p, n, &zero, c->d_cflo.p + (size_t)off * N, N));
-        }
-        off += n;
+                                     c->d_foin.p + fo.coef[s], N, c->d_tmat.p + fo.tm[s], n, &zero,
+                                     c->d_cflo.p + (size_t)off * N, N));
     }
     c->fo_done = true;
     return 0;
@@ -1201,6 +1239,7 @@ int eval_fo(flosic_ctx *c) {
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipEventRecord(c->ev[EV_START], c->stream));
     if ((r = run_frmorb(c))) return r;
+    const FoLayout fo(c);
     for (int s = 0; s < 2; ++s) {
         Spin &sp = c->sp[s];
         ALLOC(c, sp.d_ctil, (size_t)N * sp.nwf);
@@ -1209,8 +1248,8 @@ int eval_fo(flosic_ctx *c) {
             HIPCHK(c, hipMemcpyAsync(sp.d_ctil.p, c->d_cflo.p + (size_t)off * N, sizeof(double) * N * sp.nocc,
                                      hipMemcpyDeviceToDevice, c->stream));
         if (sp.nwf > sp.nocc)
-            HIPCHK(c, hipMemcpyAsync(sp.d_ctil.p + (size_t)sp.nocc * N, sp.coef.data() + (size_t)sp.nocc * N,
-                                     sizeof(double) * N * (sp.nwf - sp.nocc), hipMemcpyHostToDevice, c->stream));
+            HIPCHK(c, hipMemcpyAsync(sp.d_ctil.p + (size_t)sp.nocc * N, c->d_foin.p + fo.coef[s] + (size_t)sp.nocc * N,
+                                     sizeof(double) * N * (sp.nwf - sp.nocc), hipMemcpyDeviceToDevice, c->stream));
     }
     if ((r = ensure_planes(c))) return r;
     MARK(c, EV_FO);
@@ -1288,39 +1327,43 @@ int eval_coulomb(flosic_ctx *c) {
 // Phase C: FLOs on the mesh, XC, total potential, energies, SIC matrix and V^i_ab.  With resident planes the mesh
 // is one block; in mesh-block mode the planes, FLO fields, V_tot and U of each block are built, used and dropped,
 // and G, V^i_ab accumulate over the blocks in block order.
+// offsets (doubles) in d_res: energy sums (9 per FLO), V_H of every FLO at the outermost point, -SIC(j,i) (nwf x nocc) of both
+// spins, -SIC_ex (nocc x nocc, PBE) of both spins
+struct ResLayout {
+    size_t asy, lambda[2], lamex[2], total;
+    explicit ResLayout(const flosic_ctx *c) {
+        const size_t n0 = c->sp[0].nocc, n1 = c->sp[1].nocc, ex = c->xc == FLOSIC_XC_PBE;
+        asy = 9 * (n0 + n1);
+        lambda[0] = asy + n0 + n1;
+        lambda[1] = lambda[0] + c->sp[0].nwf * n0;
+        lamex[0] = lambda[1] + c->sp[1].nwf * n1;
+        lamex[1] = lamex[0] + ex * n0 * n0;
+        total = lamex[1] + ex * n1 * n1;
+    }
+};
 // Results of the evaluation that the host needs (energy partial sums, V_H at the outermost point, SIC(j,i), and for
 // PBE SIC_ex) queued for copying to the host on the context stream
 int queue_results(flosic_ctx *c) {
-    const int nF = c->nF;
-    c->h_energy.resize((size_t)nF * 9);
-    c->h_asy.resize(nF);
-    HIPCHK(c, hipMemcpyAsync(c->h_energy.data(), c->d_energy.p, sizeof(double) * nF * 9, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->h_asy.data(), c->d_asy.p, sizeof(double) * nF, hipMemcpyDeviceToHost, c->stream));
-    {
-        size_t lo = 0;
-        for (int s = 0; s < 2; ++s) {
-            Spin &sp = c->sp[s];
-            const int n = sp.nocc;
-            sp.sic.resize((size_t)sp.nwf * n);
-            if (n > 0)
-                HIPCHK(c, hipMemcpyAsync(sp.sic.data(), c->d_lambda.p + lo, sizeof(double) * sp.nwf * n,
-                                         hipMemcpyDeviceToHost, c->stream));
-            lo += (size_t)sp.nwf * n;
-        }
-        c->vab_on_host = false;  // V^i_ab (n^3 per spin) stays on the device until it is asked for
-    }
-    if (c->xc == FLOSIC_XC_PBE) {
-        size_t lo = 0;
-        for (int s = 0; s < 2; ++s) {
-            Spin &sp = c->sp[s];
-            const size_t nn = (size_t)sp.nocc * sp.nocc;
-            sp.sic_ex.resize(nn);
-            if (nn) HIPCHK(c, hipMemcpyAsync(sp.sic_ex.data(), c->d_lamex.p + lo, sizeof(double) * nn,
-                                             hipMemcpyDeviceToHost, c->stream));
-            lo += nn;
-        }
-    }
+    const ResLayout res(c);
+    if (!c->h_res.ensure(res.total, c->stream)) return fail(c, FLOSIC_ENOMEM, "host staging memory");
+    HIPCHK(c, hipMemcpyAsync(c->h_res.p, c->d_res.p, sizeof(double) * res.total, hipMemcpyDeviceToHost, c->stream));
+    c->vab_on_host = false;  // V^i_ab (n^3 per spin) stays on the device until it is asked for
     return 0;
+}
+// ... and, once the copy is done, put where they belong
+void take_results(flosic_ctx *c) {
+    const ResLayout res(c);
+    const double *h = c->h_res.p;
+    c->h_energy.assign(h, h + res.asy);
+    c->h_asy.assign(h + res.asy, h + res.lambda[0]);
+    for (int s = 0; s < 2; ++s) {
+        Spin &sp = c->sp[s];
+        sp.sic.assign(h + res.lambda[s], h + res.lambda[s] + (size_t)sp.nwf * sp.nocc);
+        if (c->xc == FLOSIC_XC_PBE) {
+            sp.sic_ex.resize((size_t)sp.nocc * sp.nocc);
+            for (size_t i = 0; i < sp.sic_ex.size(); ++i) sp.sic_ex[i] = -h[res.lamex[s] + i];
+        }
+    }
 }
 
 // overlap_host: with the fields resident (no mesh blocks), queue the host's results before the V^i_ab kernels so that
@@ -1337,20 +1380,15 @@ int eval_fields(flosic_ctx *c, bool overlap_host = false) {
     const int64_t mb = mesh_block(c);
     const int nblk = (int)((M + 255) / 256);
     ALLOC(c, c->d_part, (size_t)nF * nblk * 9);
-    ALLOC(c, c->d_energy, (size_t)nF * 9);
-    ALLOC(c, c->d_asy, (size_t)nF);
+    const ResLayout res(c);
+    ALLOC(c, c->d_res, res.total);
     ALLOC(c, c->d_G, (size_t)N * nF);
     ALLOC(c, c->d_phi, (size_t)nd * nF * mb);
     ALLOC(c, c->d_Vtot, (size_t)nF * mb);
     ALLOC(c, c->d_U, (size_t)nF * mb);
     if (blocked) ALLOC(c, c->d_planes, (size_t)nd * N * mb);
     const bool exact = c->xc == FLOSIC_XC_PBE;  // exact mesh derivative for the FOD gradient
-    size_t lamex_cnt = 0;
-    for (int s = 0; s < 2; ++s) lamex_cnt += (size_t)c->sp[s].nocc * c->sp[s].nocc;
-    if (exact) {
-        ALLOC(c, c->d_Ux, (size_t)4 * nF * mb);
-        ALLOC(c, c->d_lamex, lamex_cnt);
-    }
+    if (exact) ALLOC(c, c->d_Ux, (size_t)4 * nF * mb);
     size_t vab_cnt = 0, vpart_cnt = 0;
     for (int s = 0; s < 2; ++s) {
         const size_t n = (size_t)c->sp[s].nocc;
@@ -1386,14 +1424,12 @@ int eval_fields(flosic_ctx *c, bool overlap_host = false) {
         HIPCHK(c, hipGetLastError());
         if (!blocked) MARK(c, EV_XC);
         if (exact) {  // -SIC_ex(j,i) = sum_k [Ux0_i phi_j + sum_d Ux_d,i d_d phi_j], FLOs of one spin
-            size_t lo = 0;
             for (int s = 0; s < 2; ++s) {
                 const int n = c->sp[s].nocc;
                 const size_t off = s == 0 ? 0 : (size_t)n0;
-                if ((r = gemm_tn_points(c, n, n, c->d_phi.p + off * m, c->d_Ux.p + off * m, m, c->d_lamex.p + lo, k0 > 0,
-                                        0, 0, 4, (int64_t)nF * m, (int64_t)nF * m)))
+                if ((r = gemm_tn_points(c, n, n, c->d_phi.p + off * m, c->d_Ux.p + off * m, m, c->d_res.p + res.lamex[s],
+                                        k0 > 0, 0, 0, 4, (int64_t)nF * m, (int64_t)nF * m)))
                     return r;
-                lo += (size_t)n * n;
             }
         }
         // G = Phi_0^T U over the points (split K, fixed-order partial sums)
@@ -1402,24 +1438,19 @@ int eval_fields(flosic_ctx *c, bool overlap_host = false) {
         if (!defer_vab && (r = vab_all(k0, m))) return r;
     }
     if (blocked) MARK(c, EV_PHI);
-    launch_reduce_partials(c->d_part.p, nF, nblk, 9, c->d_energy.p, c->stream);
-    launch_gather(c->d_VH.p + c->kmax, M, nF, c->d_asy.p, c->stream);  // V_H of every FLO at the outermost point
+    launch_reduce_partials(c->d_part.p, nF, nblk, 9, c->d_res.p, c->stream);
+    launch_gather(c->d_VH.p + c->kmax, M, nF, c->d_res.p + res.asy, c->stream);  // V_H of every FLO at the outermost point
     if (blocked) MARK(c, EV_XC);
     // SIC_s = -Ctil_s^T G_s
-    size_t lam_cnt = 0;
-    for (int s = 0; s < 2; ++s) lam_cnt += (size_t)c->sp[s].nwf * c->sp[s].nocc;
-    ALLOC(c, c->d_lambda, lam_cnt);
     {
         const double zero = 0.0, mone = -1.0;
-        size_t lo = 0;
         for (int s = 0; s < 2; ++s) {
             Spin &sp = c->sp[s];
             const int off = s == 0 ? 0 : n0;
             if (sp.nocc > 0)
                 BLASCHK(c, rocblas_dgemm(c->blas, rocblas_operation_transpose, rocblas_operation_none, sp.nwf, sp.nocc,
                                          N, &mone, sp.d_ctil.p, N, c->d_G.p + (size_t)off * N, N, &zero,
-                                         c->d_lambda.p + lo, sp.nwf));
-            lo += (size_t)sp.nwf * sp.nocc;
+                                         c->d_res.p + res.lambda[s], sp.nwf));
         }
     }
     if (blocked) MARK(c, EV_SIC);
@@ -1444,8 +1475,7 @@ int eval_finish(flosic_ctx *c) {
         if ((r = queue_results(c))) return r;
         HIPCHK(c, hipStreamSynchronize(c->stream));
     }
-    for (int s = 0; s < 2; ++s)
-        for (double &x : c->sp[s].sic_ex) x = -x;
+    take_results(c);
     // RESULTS(1:13) per FLO (apotnl_sic.F:564-623)
     c->zsic = 0.0;
     const double e13 = (double)(1.0f / 3.0f);
@@ -2289,7 +2319,10 @@ int32_t flosic_lagmult_slv(flosic_ctx *c, int32_t ispn, const double *pot, int32
     const bool blocked = c->block_pts > 0;
     const int64_t mb = mesh_block(c);
     const int nd = xc_planes(c);
-    if ((r = upload(c, c->d_pot, pot, (size_t)M))) return r;
+    ALLOC(c, c->d_pot, (size_t)M);
+    if (!c->h_pot.ensure((size_t)M + (size_t)n * n, c->stream)) return fail(c, FLOSIC_ENOMEM, "host staging memory");
+    std::copy(pot, pot + M, c->h_pot.p);  // the previous call has waited for its result, which lies behind its copy
+    HIPCHK(c, hipMemcpyAsync(c->d_pot.p, c->h_pot.p, sizeof(double) * M, hipMemcpyHostToDevice, c->stream));
     ALLOC(c, c->d_lap, (size_t)(nd == 10 ? 3 : 1) * n * mb);
     ALLOC(c, c->d_wop, (size_t)n * mb);
     ALLOC(c, c->d_small, (size_t)n * n);
@@ -2325,8 +2358,8 @@ int32_t flosic_lagmult_slv(flosic_ctx *c, int32_t ispn, const double *pot, int32
         HIPCHK(c, hipGetLastError());
         if ((r = gemm_tn_points(c, n, n, phi, c->d_wop.p, m, c->d_small.p, k0 > 0))) return r;
     }
-    std::vector<double> L((size_t)n * n);
-    HIPCHK(c, hipMemcpyAsync(L.data(), c->d_small.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, c->stream));
+    double *L = c->h_pot.p + M;
+    HIPCHK(c, hipMemcpyAsync(L, c->d_small.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     for (int k = 0; k < n; ++k)
         for (int j = 0; j < n; ++j) sic[j + (size_t)ldsic * k] += L[j + (size_t)n * k];
