@@ -28,7 +28,7 @@ namespace flosic {
 //
 // Measured on synthetic systems (kernel time, against one 16-wave block per tile with dedicated R, copy and consumer
 // waves that met at a barrier every 16 or 32 rows, columns padded to 64): FP64 30 FLOs / 116 200 points / 1686 groups
-// 7.64 -> 2.36 ms; 48 / 185 742 / 4163 32.6 -> 12.6 ms (57 TFLOP/s, 74% of the 77.5 that FP64 MFMAs alone reach);
+// 7.64 -> 2.24 ms; 48 / 185 742 / 4163 32.6 -> 12.3 ms (59 TFLOP/s, 76% of the 77.5 that FP64 MFMAs alone reach);
 // 96 / 370 513 / 15 750 311 -> 173 ms; 192 / 196 174 / 60 795 784 -> 625 ms (82%).  FP32: 3.26 -> 1.21, 13.9 -> 7.1,
 // 162 -> 91, 415 -> 338 ms (74% of 158 TFLOP/s).
 //
