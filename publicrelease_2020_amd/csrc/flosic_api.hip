@@ -899,7 +899,6 @@ int ensure_planes(flosic_ctx *c) {
     if (c->block_pts > 0 || (c->planes_ok && c->planes_nd == nd)) return 0;
     const size_t cnt = (size_t)nd * c->nbas * (size_t)c->M;
     ALLOC(c, c->d_planes, cnt);
-    HIPCHK(c, hipMemsetAsync(c->d_planes.p, 0, cnt * sizeof(double), c->stream));
     launch_basis_planes<double>(basis_view(c), c->d_x.p, c->d_y.p, c->d_z.p, c->M, nd, c->d_planes.p, c->M, c->stream);
     HIPCHK(c, hipGetLastError());
     c->planes_nd = nd;
@@ -909,8 +908,6 @@ int ensure_planes(flosic_ctx *c) {
 
 // Basis planes of the mesh block [k0, k0 + m) into dst (leading dimension m); nd as launch_basis_planes
 int block_planes(flosic_ctx *c, int64_t k0, int64_t m, int nd, double *dst) {
-    const size_t cnt = (size_t)(nd == -1 ? 1 : nd == -3 ? 3 : nd) * c->nbas * (size_t)m;
-    launch_fill_zero(dst, cnt, c->stream);  // a kernel, not a memset node, so that the block loop can be captured
     launch_basis_planes<double>(basis_view(c), c->d_x.p + k0, c->d_y.p + k0, c->d_z.p + k0, m, nd, dst, m, c->stream);
     HIPCHK(c, hipGetLastError());
     return 0;
@@ -973,10 +970,8 @@ int run_frmorb(flosic_ctx *c) {
     for (int s = 0; s < 2; ++s) std::copy(c->sp[s].coef.begin(), c->sp[s].coef.end(), h_in + fo.coef[s]);
     HIPCHK(c, hipMemcpyAsync(c->d_foin.p, h_in, sizeof(double) * fo.total, hipMemcpyHostToDevice, c->stream));
     // chi planes [K][mu][FOD], K = value, d/dx, d/dy, d/dz
-    launch_fill_zero(c->d_fodchi.p, 4 * (size_t)N * nfod, c->stream);
-    if (nfod > 0)
-        launch_basis_planes<double>(basis_view(c), c->d_foin.p, c->d_foin.p + nfod, c->d_foin.p + 2 * nfod, nfod, 4,
-                                    c->d_fodchi.p, nfod, c->stream);
+    launch_basis_planes<double>(basis_view(c), c->d_foin.p, c->d_foin.p + nfod, c->d_foin.p + 2 * nfod, nfod, 4,
+                                c->d_fodchi.p, nfod, c->stream);
     HIPCHK(c, hipGetLastError());
     const double one = 1.0, zero = 0.0;
     for (int s = 0, off = 0; s < 2; off += c->sp[s].nocc, ++s) {
