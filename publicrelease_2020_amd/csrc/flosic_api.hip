@@ -2161,10 +2161,7 @@ int32_t flosic_siclag_der(flosic_ctx *c, double *dersic) {
     const bool blocked = c->block_pts > 0;
     ALLOC(c, c->d_dG, (size_t)3 * N * nF);
     if (!blocked && nd == 10) {  // resident PBE planes: value, gradient, Hessian of every function on the mesh
-        for (int d = 0; d < 3; ++d)
-            if ((r = gemm_tn_points(c, N, nF, c->d_planes.p + (size_t)(1 + d) * N * M, c->d_U.p, M,
-                                    c->d_dG.p + (size_t)d * N * nF)))
-                return r;
+        if ((r = gemm_tn_points(c, 3 * N, nF, c->d_planes.p + (size_t)N * M, c->d_U.p, M, c->d_dG.p))) return r;
     } else {
         const int64_t mb = blocked ? mesh_block(c) : std::min<int64_t>(M, kDerBlockPts);
         const int nblk = (int)((M + 255) / 256);
@@ -2189,10 +2186,8 @@ int32_t flosic_siclag_der(flosic_ctx *c, double *dersic) {
                 u = c->d_du.p;
                 ldu = m;
             }
-            for (int d = 0; d < 3; ++d)
-                if ((r = gemm_tn_points(c, N, nF, c->d_dplanes.p + (size_t)(g0 + d) * N * m, u, m,
-                                        c->d_dG.p + (size_t)d * N * nF, k0 > 0, m, ldu)))
-                    return r;
+            if ((r = gemm_tn_points(c, 3 * N, nF, c->d_dplanes.p + (size_t)g0 * N * m, u, m, c->d_dG.p, k0 > 0, m, ldu)))
+                return r;
         }
     }
     std::vector<double> G((size_t)3 * N * nF), cf((size_t)N * nF);
@@ -2204,7 +2199,7 @@ int32_t flosic_siclag_der(flosic_ctx *c, double *dersic) {
         const int f0 = c->fstart[3 * a], f1 = a + 1 < c->natom ? c->fstart[3 * (a + 1)] : N;
         for (int i = 0; i < nF; ++i)
             for (int x = 0; x < 3; ++x) {
-                const double *g = G.data() + (size_t)x * N * nF + (size_t)N * i;
+                const double *g = G.data() + (size_t)N * (x + 3 * (size_t)i);  // the planes stack: 3 N rows per FLO
                 double acc = 0.0;
                 for (int f = f0; f < f1; ++f) acc -= cf[f + (size_t)N * i] * g[f];
                 dersic[x + 3 * ((size_t)i + (size_t)nF * a)] = fac * acc;
