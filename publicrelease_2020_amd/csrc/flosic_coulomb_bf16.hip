@@ -19,17 +19,21 @@ namespace flosic {
 //                   by themselves for four runs of chunks, and meet in the final sum.  No barrier in the loop.
 //   up to  96 FLOs  CW = 2: two tiles of 64 points; up to 192 FLOs CW = 4: one tile.  More FLOs: further blocks.
 // With CW > 1 the waves have roles, because the sums leave no room for both R and H operands loaded ahead (waves that did
-// everything in turn ran 192 FLOs, 5.2e5 rows, 2.0e5 points at 272 ms, the registers spilling, against 210 ms with roles):
+// everything in turn ran 192 FLOs, 5.2e5 rows, 2.0e5 points at 272 ms, the registers spilling, against 192 ms with roles):
 // waves 0-3 are consumers, CW on each tile, whose H operands are loaded one K step ahead; waves 4-7 producers, CW on each
-// tile.  While the consumers run the MFMAs of chunk c, the producers split R of chunk c + 1 into A operands and make R of
-// chunk c + 2 (FP32, lane = point), both in two LDS buffers; one barrier per chunk of 64 Hermite rows.
+// tile.  While the consumers run the MFMAs of chunk c, the producers work ahead, one barrier per chunk of 64 Hermite rows.
+// CW = 2: they split R of chunk c + 1 into A operands and make R of chunk c + 2 (FP32, lane = point), both in two LDS
+// buffers.  CW = 4: they make R of a pair of chunks in one phase (two, three or six groups of L = 4, 3, 2 do not share out over
+// four waves, twice as many do) and split the pair in the next, A operands in three buffers.  The producers have the
+// higher wave priority: their VALU instructions fit beside the consumer's MFMAs, and a late producer holds up all.
 // The FP32 accumulators go into the FP64 sums at the chunks marked flush (every 256 or more rows), so the sums do not
 // depend on the split.
 // Measured, three pieces, against 16-wave blocks in which two waves of every block staged H through LDS: 10 FLOs (289 groups,
-// 3.4e4 points) 0.279 -> 0.126 ms; 30 FLOs (1686, 1.2e5) 2.98 -> 1.24; 48 FLOs (4163, 1.9e5) 12.6 -> 5.5; 64 FLOs (7371,
-// 2.4e5) 25.8 -> 20.5; 96 FLOs (15750, 3.7e5) 96.0 -> 76.2; 120 FLOs (24241, 3.1e5) 104 -> 93.7; 144 FLOs (33810, 2.8e5)
-// 162 -> 121; 192 FLOs (60795, 2.0e5) 242 -> 210.  With CW = 1 making R bounds the loop (32 and 48 FLOs take the same time per
-// row and point); with CW = 4 the MFMAs are 52% busy, producers alone take 140 ms of the 210 and consumers alone 170.
+// 3.4e4 points) 0.279 -> 0.125 ms; 30 FLOs (1686, 1.2e5) 2.98 -> 1.18; 48 FLOs (4163, 1.9e5) 12.6 -> 5.1; 64 FLOs (7371,
+// 2.4e5) 25.8 -> 17.5; 96 FLOs (15750, 3.7e5) 96.0 -> 68.2; 120 FLOs (24241, 3.1e5) 104 -> 85.5; 192 FLOs (60795, 2.0e5)
+// 242 -> 192.  With CW = 1 making R bounds the loop (32 and 48 FLOs take nearly the same time per row and point).  With
+// CW = 4 the MFMAs are 57% busy: of the 192 ms the MFMAs alone need 111, with A from LDS 118, with the FP64 sums 130, with
+// H from L2 (three quarters of a gigabyte per tile, 96% hits) 168; the rest is what the producers take from the consumers.
 // ---------------------------------------------------------------------------------------------------
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v2f __attribute__((ext_vector_type(2)));
@@ -179,7 +183,7 @@ __device__ __forceinline__ int r_at(int point, int row) {
 template <int NP, int CW>
 struct BfTile {                         // LDS of one 64-point tile with CW > 1
     float R[2][bf_rsize<CW == 4>];
-    v8bf A[2][2][4][NP][64];            // A operands [buffer][K step][point tile][piece][lane]
+    v8bf A[CW == 4 ? 3 : 2][2][4][NP][64];  // A operands [buffer][K step][point tile][piece][lane]
 };
 constexpr int kBfTab = kBoysRows * kBoysCols * 4;  // the FP32 Boys table, in LDS with CW = 4
 template <int NP, int CW>
@@ -236,24 +240,32 @@ __device__ __forceinline__ void hermite_Rn(const float *p, const float (*X)[3], 
     }
 }
 
-// R of NG groups of a chunk, g0 and g0 + step (rows RPG g .. of the chunk hold rows ROFF .. of group g), for this lane's
-// point
+// Consecutive groups of one chunk type, [pb, pb + np): those from np0 on belong to the next chunk, whose R lies bf_rsize
+// further.  P: the records of the first two this wave makes (bf_records).
+struct BfGroups {
+    int type, pb, np, np0;
+};
+__device__ __forceinline__ v4d bf_record(const double4 *__restrict__ pP, const BfGroups &G, int g) {
+    return cload(reinterpret_cast<const v4d *>(pP + G.pb + min(g, G.np - 1)));
+}
+// R of NG groups, g0 and g0 + step (rows RPG g .. of the chunk hold rows ROFF .. of its group g), for this lane's point; P
+// their centres and exponents
 template <bool PAD, int L, int RPG, int ROFF, int NG>
-__device__ __forceinline__ void bf_groups(const double4 *__restrict__ pP, int g0, int step, int lane, double px, double py,
-                                          double pz, const float *__restrict__ tab, float *__restrict__ R) {
+__device__ __forceinline__ void bf_groups(const v4d *P, const BfGroups &G, int g0, int step, int lane, double px, double py, double pz,
+                                          const float *__restrict__ tab, float *__restrict__ R0) {
     float p[NG], X[NG][3], r[NG][ntuv(L)];
 #pragma unroll
     for (int e = 0; e < NG; ++e) {
-        const v4d P = cload(reinterpret_cast<const v4d *>(pP + g0 + e * step));
-        p[e] = (float)P.w;
-        X[e][0] = (float)(P.x - px);
-        X[e][1] = (float)(P.y - py);
-        X[e][2] = (float)(P.z - pz);
+        p[e] = (float)P[e].w;
+        X[e][0] = (float)(P[e].x - px);
+        X[e][1] = (float)(P[e].y - py);
+        X[e][2] = (float)(P[e].z - pz);
     }
     hermite_Rn<L, NG, ROFF == 32>(p, X, tab, r);
 #pragma unroll
     for (int e = 0; e < NG; ++e) {
-        const int row0 = (g0 + e * step) * RPG;
+        const int ge = g0 + e * step, row0 = (ge < G.np0 ? ge : ge - G.np0) * RPG;
+        float *__restrict__ R = R0 + (ge < G.np0 ? 0 : bf_rsize<PAD>);
         if constexpr (RPG % 4 == 0) {
 #pragma unroll
             for (int t = 0; t < RPG; t += 4)
@@ -268,31 +280,36 @@ __device__ __forceinline__ void bf_groups(const double4 *__restrict__ pP, int g0
         }
     }
 }
-// groups first, first + step, ... of the chunk, two at a time
+// groups first, first + step, ..., two at a time, the next two's records on their way meanwhile
 template <bool PAD, int L, int RPG = ntuv(L), int ROFF = 0>
-__device__ __forceinline__ void bf_chunk_R(const ChunkDev &ch, int first, int step, const double4 *__restrict__ pP,
-                                           int lane, double px, double py, double pz, const float *__restrict__ tab,
-                                           float *__restrict__ R) {
-    const int np = ch.pe - ch.pb;
+__device__ __forceinline__ void bf_chunk_R(const BfGroups &G, int first, int step, const double4 *__restrict__ pP,
+                                           v4d (&P)[2], int lane, double px, double py, double pz,
+                                           const float *__restrict__ tab, float *__restrict__ R) {
     int g = first;
-    for (; g + step < np; g += 2 * step)
-        bf_groups<PAD, L, RPG, ROFF, 2>(pP + ch.pb, g, step, lane, px, py, pz, tab, R);
-    if (g < np) bf_groups<PAD, L, RPG, ROFF, 1>(pP + ch.pb, g, step, lane, px, py, pz, tab, R);
+    for (; g + step < G.np; g += 2 * step) {
+        const v4d Q[2] = {bf_record(pP, G, g + 2 * step), bf_record(pP, G, g + 3 * step)};
+        __builtin_amdgcn_sched_barrier(0);
+        bf_groups<PAD, L, RPG, ROFF, 2>(P, G, g, step, lane, px, py, pz, tab, R);
+        P[0] = Q[0];
+        P[1] = Q[1];
+    }
+    if (g < G.np) bf_groups<PAD, L, RPG, ROFF, 1>(P, G, g, step, lane, px, py, pz, tab, R);
 }
 
 template <bool PAD>
-__device__ __forceinline__ void bf_make_R(const ChunkDev &ch, int first, int step, const double4 *__restrict__ pP, int lane,
-                                          double px, double py, double pz, const float *__restrict__ tab,
-                                          float *__restrict__ R) {
-    switch (ch.L) {
-        case 0: bf_chunk_R<PAD, 0>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
-        case 1: bf_chunk_R<PAD, 1>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
-        case 2: bf_chunk_R<PAD, 2>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
-        case 3: bf_chunk_R<PAD, 3>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
-        case 5: bf_chunk_R<PAD, 4, chunk_rpg(5), chunk_roff(5)>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
-        default: bf_chunk_R<PAD, 4, chunk_rpg(6), chunk_roff(6)>(ch, first, step, pP, lane, px, py, pz, tab, R); break;
+__device__ __forceinline__ void bf_make_R(const BfGroups &G, int first, int step, const double4 *__restrict__ pP,
+                                          v4d (&P)[2], int lane, double px, double py, double pz,
+                                          const float *__restrict__ tab, float *__restrict__ R) {
+    switch (G.type) {
+        case 0: bf_chunk_R<PAD, 0>(G, first, step, pP, P, lane, px, py, pz, tab, R); break;
+        case 1: bf_chunk_R<PAD, 1>(G, first, step, pP, P, lane, px, py, pz, tab, R); break;
+        case 2: bf_chunk_R<PAD, 2>(G, first, step, pP, P, lane, px, py, pz, tab, R); break;
+        case 3: bf_chunk_R<PAD, 3>(G, first, step, pP, P, lane, px, py, pz, tab, R); break;
+        case 5: bf_chunk_R<PAD, 4, chunk_rpg(5), chunk_roff(5)>(G, first, step, pP, P, lane, px, py, pz, tab, R); break;
+        default: bf_chunk_R<PAD, 4, chunk_rpg(6), chunk_roff(6)>(G, first, step, pP, P, lane, px, py, pz, tab, R); break;
     }
 }
+__device__ __forceinline__ BfGroups bf_chunk_groups(const ChunkDev &c) { return BfGroups{c.L, c.pb, c.pe - c.pb, c.pe - c.pb}; }
 // rows 32 q + 8 lr .. + 7 of point 16 i + lc, split
 template <int NP, bool PAD>
 __device__ __forceinline__ void bf_rows8(const float *R, int i, int q, int lr, int lc, v8bf (&a)[NP]) {
@@ -327,15 +344,14 @@ struct BfAcc {
                 }
     }
     // one K step: products of the pieces in the order a0b0, a0b1, a1b0 (a0b2, a1b1, a2b0) for every accumulator, one point
-    // tile after the other.  next_a(i, a) gives the A operand of tile i; it is issued before the MFMAs of tile i - 1 and,
-    // with HOLD, the scheduler is kept from moving it down to its use.
+    // tile after the other.  next_a(i, a) gives the A operand of tile i, i = 4: of the next K step's tile 0 (or nothing);
+    // it is issued before the MFMAs of tile i - 1 and, with HOLD, the scheduler is kept from moving it down to its use.
+    // a[0]: the operand of tile 0.
     template <bool HOLD, typename F>
-    __device__ __forceinline__ void step(F next_a, const v8bf (&b)[NT][NP]) {
-        v8bf a[2][NP];
-        next_a(0, a[0]);
+    __device__ __forceinline__ void step(v8bf (&a)[2][NP], F next_a, const v8bf (&b)[NT][NP]) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            if (i < 3) next_a(i + 1, a[(i + 1) & 1]);
+            next_a(i + 1, a[(i + 1) & 1]);
             if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);
 #define FLOSIC_BF(pa, pb)                          \
     _Pragma("unroll") for (int j = 0; j < NT; ++j) \
@@ -459,13 +475,20 @@ __device__ __forceinline__ void bf_alone(unsigned char *__restrict__ lds, const 
         int flush;
         do {
         const ChunkDev ch = chunk_at(J.chunks, c);
-        bf_make_R<true>(ch, 0, 1, J.pP, lane, P.x, P.y, P.z, ctab, R);
+        __builtin_amdgcn_s_setprio(0);
+        v4d rec[2] = {bf_record(J.pP, bf_chunk_groups(ch), 0), bf_record(J.pP, bf_chunk_groups(ch), 1)};
+        bf_make_R<true>(bf_chunk_groups(ch), 0, 1, J.pP, rec, lane, P.x, P.y, P.z, ctab, R);
+        __builtin_amdgcn_s_setprio(2);  // the MFMA half goes first (30 FLOs 1.26 -> 1.18 ms, 48 FLOs 5.26 -> 5.07)
         wave_lds_sync();
         const bool f = bf_far<NP>(far, c);
 #pragma unroll 1
         for (int q = 0; q < 2; ++q) {
-            auto next_a = [&](int i, v8bf(&a)[NP]) { bf_rows8<NP, true>(R, i, q, lr, lc, a); };
-            A.template step<true>(next_a, b);
+            auto next_a = [&](int i, v8bf(&x)[NP]) {
+                if (i < 4) bf_rows8<NP, true>(R, i, q, lr, lc, x);
+            };
+            v8bf a[2][NP];
+            next_a(0, a[0]);
+            A.template step<true>(a, next_a, b);
             h += hstep;
             if (q == 0) bf_load<NP, NT>(b, h, pstride, f, zero);
             else if (c + 1 < c1) bf_load<NP, NT>(b, h, pstride, bf_far<NP>(far, c + 1), zero);
@@ -482,36 +505,89 @@ __device__ __forceinline__ void bf_alone(unsigned char *__restrict__ lds, const 
 template <int NP, int CW>
 __device__ __forceinline__ void bf_producer(BfTile<NP, CW> &T, const CoulJob<__bf16> &J, const float *__restrict__ ctab,
                                             int64_t tile, int pi, int ntmax) {
+    constexpr bool PAD = CW == 4;
     const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15;
     const BfPoint P = bf_point(J, tile);
     const int n = J.nchunks;
+    __builtin_amdgcn_s_setprio(2);  // a producer's VALU instructions go into the cycles in which the consumer's MFMA runs
     // rows of a chunk beyond its groups are never written and meet zero rows of H: they only have to be finite
-    for (int i = pi * 64 + lane; i < bf_rsize<CW == 4> / 2; i += 64 * CW) ((v4f *)T.R[0])[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = pi * 64 + lane; i < bf_rsize<PAD> / 2; i += 64 * CW) ((v4f *)T.R[0])[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     role_barrier();
-    auto make = [&](int c) {  // which producer begins changes from chunk to chunk
-        bf_make_R<CW == 4>(chunk_at(J.chunks, c), (pi + c) % CW, CW, J.pP, lane, P.x, P.y, P.z, ctab, T.R[c & 1]);
-    };
-    auto split = [&](int c) {
+    auto split = [&](int c, int slot) {
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int e = 0; e < 4 / CW; ++e) {
                 const int i = pi * (4 / CW) + e;
                 v8bf a[NP];
-                bf_rows8<NP, CW == 4>(T.R[c & 1], i, q, lr, lc, a);
+                bf_rows8<NP, PAD>(T.R[c & 1], i, q, lr, lc, a);
 #pragma unroll
-                for (int p = 0; p < NP; ++p) T.A[c & 1][q][i][p][lane] = a[p];
+                for (int p = 0; p < NP; ++p) T.A[slot][q][i][p][lane] = a[p];
             }
     };
-    make(0);
-    role_barrier();
-    split(0);
-    if (n > 1) make(1);
-    role_barrier();
-    for (int c = 0; c < n; ++c) {
-        if (c + 1 < n) split(c + 1);
-        if (c + 2 < n) make(c + 2);
+    if constexpr (CW == 4) {  // chunks in pairs (even, odd): R of a pair in one phase, its split in the next
+        BfGroups G[2];
+        v4d rec[2];
+        int parts;
+        auto plan = [&](int c) {  // the groups of chunks c and c + 1, in one list where they follow one another
+            const ChunkDev x = chunk_at(J.chunks, c);
+            G[0] = G[1] = bf_chunk_groups(x);
+            parts = 1;
+            if (c + 1 < n) {
+                const ChunkDev y = chunk_at(J.chunks, c + 1);
+                if (y.L == x.L && y.pb == x.pe) {
+                    G[0].np += y.pe - y.pb;
+                } else {
+                    G[1] = bf_chunk_groups(y);
+                    parts = 2;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 2; ++e) rec[e] = bf_record(J.pP, G[0], pi + 4 * e);
+        };
+        auto make = [&]() {
+            bf_make_R<PAD>(G[0], pi, 4, J.pP, rec, lane, P.x, P.y, P.z, ctab, T.R[0]);
+            if (parts == 2) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) rec[e] = bf_record(J.pP, G[1], 3 - pi + 4 * e);
+                bf_make_R<PAD>(G[1], 3 - pi, 4, J.pP, rec, lane, P.x, P.y, P.z, ctab, T.R[1]);
+            }
+        };
+        plan(0);
+        make();
         role_barrier();
+        split(0, 0);
+        if (n > 1) split(1, 1);
+        if (n > 2) plan(2);
+        role_barrier();
+        for (int c = 0, slot = 0; c < n; ++c) {  // slot = c % 3
+            slot = slot == 2 ? 0 : slot + 1;
+            if (c & 1) {
+                if (c + 1 < n) split(c + 1, slot);
+                if (c + 2 < n) split(c + 2, slot == 2 ? 0 : slot + 1);
+                if (c + 3 < n) plan(c + 3);
+            } else if (c + 2 < n) {
+                make();
+            }
+            role_barrier();
+        }
+    } else {
+        auto make = [&](int c) {  // which producer begins changes from chunk to chunk
+            const BfGroups G = bf_chunk_groups(chunk_at(J.chunks, c));
+            const int first = (pi + c) % CW;
+            v4d rec[2] = {bf_record(J.pP, G, first), bf_record(J.pP, G, first + CW)};
+            bf_make_R<PAD>(G, first, CW, J.pP, rec, lane, P.x, P.y, P.z, ctab, T.R[c & 1]);
+        };
+        make(0);
+        role_barrier();
+        split(0, 0);
+        if (n > 1) make(1);
+        role_barrier();
+        for (int c = 0; c < n; ++c) {
+            if (c + 1 < n) split(c + 1, (c + 1) & 1);
+            if (c + 2 < n) make(c + 2);
+            role_barrier();
+        }
     }
     for (int j = 0; j < ntmax; ++j) {  // the consumers' epilogue
         __syncthreads();
@@ -534,28 +610,32 @@ __device__ __forceinline__ void bf_consumer(unsigned char *__restrict__ lds, BfT
     bool f = bf_far<NP>(far, 0);
     bf_load<NP, NT>(b0, h, pstride, f, zero);
     bf_load<NP, NT>(b1, h + hstep, pstride, f, zero);
-    __builtin_amdgcn_s_setprio(2);  // MFMAs first, the producer beside them fills the gaps
     role_barrier();
     role_barrier();
     role_barrier();
-    for (int c = 0; c < n;) {
+    for (int c = 0, slot = 0; c < n;) {  // slot = c % 2 or 3
         int flush;
         do {  // up to the next flush, which the last chunk has: the sums are not live across a branch
         const bool more = c + 1 < n, fn = more && bf_far<NP>(far, c + 1);
         flush = __builtin_amdgcn_readfirstlane(cload(&J.chunks[c].flush));
         if (more) h += 2 * hstep;  // the last chunk's are loaded again
-        auto a0 = [&](int i, v8bf(&a)[NP]) {
+        const auto &As = T.A[slot];
+        auto a0 = [&](int i, v8bf(&x)[NP]) {
 #pragma unroll
-            for (int p = 0; p < NP; ++p) a[p] = T.A[c & 1][0][i][p][lane];
+            for (int p = 0; p < NP; ++p) x[p] = As[i >> 2][i & 3][p][lane];
         };
-        auto a1 = [&](int i, v8bf(&a)[NP]) {
+        auto a1 = [&](int i, v8bf(&x)[NP]) {
 #pragma unroll
-            for (int p = 0; p < NP; ++p) a[p] = T.A[c & 1][1][i][p][lane];
+            for (int p = 0; p < NP; ++p)
+                if (i < 4) x[p] = As[1][i & 3][p][lane];
         };
-        A.template step<CW == 4>(a0, b0);
+        v8bf a[2][NP];
+        a0(0, a[0]);
+        A.template step<CW == 4>(a, a0, b0);
         bf_load<NP, NT>(b0, h, pstride, fn, zero);
-        A.template step<CW == 4>(a1, b1);
+        A.template step<CW == 4>(a, a1, b1);
         bf_load<NP, NT>(b1, h + hstep, pstride, fn, zero);
+        slot = slot == (CW == 4 ? 2 : 1) ? 0 : slot + 1;
         f = fn;
         ++c;
         role_barrier();
