@@ -1388,7 +1388,7 @@ int eval_fields(flosic_ctx *c, bool overlap_host = false) {
     for (int s = 0; s < 2; ++s) {
         const size_t n = (size_t)c->sp[s].nocc;
         vab_cnt += n * n * n;
-        vpart_cnt = std::max(vpart_cnt, (size_t)vab_slices(mb) * n * n * n);
+        vpart_cnt = std::max(vpart_cnt, (size_t)vab_slices(mb, (int)n) * n * n * n);
     }
     ALLOC(c, c->d_vab, vab_cnt);
     ALLOC(c, c->d_vabpart, vpart_cnt);
@@ -1399,7 +1399,7 @@ int eval_fields(flosic_ctx *c, bool overlap_host = false) {
             const int n = c->sp[s].nocc;
             if (n == 0) continue;
             const int off = s == 0 ? 0 : n0;
-            const int nsl = vab_slices(m);
+            const int nsl = vab_slices(m, n);
             launch_vab(c->d_phi.p + (size_t)off * m, c->d_Vtot.p + (size_t)off * m, c->d_w.p + k0, m, n, nsl,
                        c->d_vabpart.p, c->stream, c->prec != FLOSIC_PREC_FP64);
             HIPCHK(c, hipGetLastError());

@@ -1201,11 +1201,15 @@ __global__ void __launch_bounds__(256) k_vab_mfma(const double *__restrict__ phi
         }
 }
 
-int vab_slices(int64_t M) {
-    // point slices per spin: enough blocks to fill the chip, slices of at least 1024 points
+// Point slices: at least 64 where they have 1024 points each; for few FLOs, whose pair blocks are few, as many as give 1024
+// blocks in all, of at least 256 points (eight staged steps).  With 64 at most, 10 FLOs (one pair block per spin, 3.4e4
+// points) took 24 us per spin, 48 FLOs in FP32 (six, 1.9e5 points) 118; now 8.7 and 80.
+int vab_slices(int64_t M, int n) {
     int s = 64;
     while (s > 1 && M / s < 1024) --s;
-    return s;
+    const int64_t nb8 = (n + 7) / 8, per_slice = nb8 * (nb8 + 1) / 2 * ((n + 127) / 128);
+    const int64_t more = std::min<int64_t>(1024 / std::max<int64_t>(1, per_slice), M / 256);
+    return (int)std::max<int64_t>(s, more);
 }
 
 void launch_vab(const double *phi0, const double *Vtot, const double *w, int64_t M, int n, int nslice, double *part,
