@@ -33,17 +33,12 @@ PEAK = {"fp64": ("f64", 78.6), "mixed": ("f32", 157.3), "bf16x3": ("bf16", 2500.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "coulomb_k64_traffic.txt")
 
 
-def coulomb_kernel_name(prec: str, nF: int, cols: int = 0) -> str:
-    """Name of the Coulomb kernel instantiation the library launches for this form, FLO count and tile width
-    (0: the widest, the library's default)."""
-    if cols <= 0:
-        cols = 64 if nF <= 64 else 128 if nF <= 128 else 192 if nF <= 192 else 256
-    if prec == "fp64":
-        return f"k_coulomb_ws<double, {cols}>"
-    if prec == "mixed":
-        return f"k_coulomb_ws<float, {cols}>"
-    npc = 3 if prec == "bf16x3" else 2
-    return f"k_coulomb_ws_bf16<{npc}, {min(cols, 192) if cols != 256 else 128}>"
+def coulomb_kernel_name(prec: str) -> str:
+    """Name of the Coulomb kernel template that the library launches for this form (its further arguments, the split over
+    waves, follow from the FLO count)."""
+    if prec in ("fp64", "mixed"):
+        return f"k_coulomb_fp<{'double' if prec == 'fp64' else 'float'}>"
+    return f"k_coulomb_bf16<{3 if prec == 'bf16x3' else 2}>"
 
 
 def measured_traffic(kernel: str, atoms: int):
@@ -433,7 +428,7 @@ def bench_batch(args) -> int:
         "peak_device_bytes": int(peak),
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK[form][1], "unit": "TFLOP/s",
                      "frac": achieved / PEAK[form][1], "traffic": None,
-                     "kernel": ("k_coulomb_ws_batch_all<float>" if form == "mixed" else "k_coulomb_ws_bf16_batch_all<*>"),
+                     "kernel": ("k_coulomb_fp_batch_all<float>" if form == "mixed" else "k_coulomb_bf16_batch_all<*>"),
                      "kernel_ms": t_eager[2],
                      "flops_per_launch": flops, "one_at_a_time_kernel_ms": seq_coul},
     }
@@ -577,7 +572,7 @@ def main() -> int:
     best = max(ok, key=lambda r: r["evals_s"]) if ok else ref
     flops = coulomb_flops(best["counts"])
     arith, peak = PEAK[best["prec"]]
-    kname = coulomb_kernel_name(best["prec"], int(best["counts"][4]), int(best["counts"][8]))
+    kname = coulomb_kernel_name(best["prec"])
     # compulsory HBM bytes of one launch: H once in the form's operand layout, V written once, mesh coordinates
     c = best["counts"]
     hbytes = {"fp64": 8, "mixed": 4, "bf16x3": 6, "bf16x2": 4}[best["prec"]]

@@ -930,10 +930,6 @@ int check_ready(flosic_ctx *c) {
     return 0;
 }
 
-// FRMORB2(0,0) + FRMIORB(1,1) for both spins: the basis and its gradient at every FOD (the mesh basis kernel with the
-// FODs of both spins as its points), Psi_K = C^T chi_K at the FODs (4 products of nocc x nbas x nocc per spin,
-// rocBLAS), the n x n Lowdin algebra of the two spins on two host threads, then cflo = C_occ TMAT^T (rocBLAS); the FLO
-// coefficients of all FLOs land in d_cflo (nbas x nF, spin 1 first)
 // offsets (doubles) in d_foin: 3 x nfod coordinates, then C (nbas x nwf) of both spins; in d_tmat: n x n of both spins
 struct FoLayout {
     size_t coef[2], tm[2], total, ntm;
@@ -947,6 +943,10 @@ struct FoLayout {
         ntm = tm[1] + n1 * n1;
     }
 };
+// FRMORB2(0,0) + FRMIORB(1,1) for both spins: the basis and its gradient at every FOD (the mesh basis kernel with the
+// FODs of both spins as its points), Psi_K = C^T chi_K at the FODs (4 products of nocc x nbas x nocc per spin,
+// rocBLAS), the n x n Lowdin algebra of the two spins on two host threads, then cflo = C_occ TMAT^T (rocBLAS); the FLO
+// coefficients of all FLOs land in d_cflo (nbas x nF, spin 1 first)
 int run_frmorb(flosic_ctx *c) {
     const int N = c->nbas;
     const int n0 = c->sp[0].nocc, nfod = n0 + c->sp[1].nocc;

@@ -186,8 +186,8 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 // Loads and stores through a pointer typed as global memory.  The batch kernels read their arrays' addresses from a
 // job table in device memory, and to the compiler such an address is generic: accesses through it become flat
-// instructions, which also count against the LDS counter, so a copy wave's wait for its LDS stores would drain its
-// global loads in flight as well.  The Coulomb tiles load and store through these (with scalar or ext_vector
+// instructions, which also count against the LDS counter, so a wait for LDS would drain the wave's global loads in
+// flight as well.  The Coulomb tiles load and store through these (with scalar or ext_vector
 // types: a class type such as double4 would be copied through its generic-address copy constructor).
 template <typename T>
 __device__ __forceinline__ T gload(const T *p) {
@@ -199,7 +199,7 @@ __device__ __forceinline__ void gstore(T *p, T v) {
 }
 // Load of read-only data at a wave-uniform address through the constant address space: a scalar load (lgkm
 // counter), which leaves the wave's vector loads in flight.  A vector load there would need a vmcnt wait before
-// its value could be made uniform, draining the copy waves' H loads with it.
+// its value could be made uniform, draining the H loads in flight with it.
 template <typename T>
 __device__ __forceinline__ T cload(const T *p) {
     return *(const __attribute__((address_space(4))) T *)p;
