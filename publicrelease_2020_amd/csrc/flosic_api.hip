@@ -186,7 +186,7 @@ struct flosic_ctx {
     DevBuf<double> d_ps_coef;
     DevBuf<PairDev> d_pairs;
     DevBuf<ChunkDev> d_chunks_bf16;
-    int nchunks_bf16 = 0, rgc_bf16[5] = {0, 0, 0, 0, 0};  // chunks and the four runs of them (CoulJob)
+    int nchunks_bf16 = 0, rgc_bf16[kRunsBf16 + 1] = {};  // chunks and the runs of them (CoulJob)
     int64_t rows_padded = 0, rows_padded_bf16 = 0;  // Hermite rows as the FP and the split-BF16 kernels stream them
     DevBuf<double> d_lapplane, d_lap, d_pot, d_wop, d_small, d_B, d_hao;  // LAGMULT_SLV / AO SIC Hamiltonian
     DevBuf<double> d_scf;  // SCFSICW orbital update: ham_ao, ham_ao C, C^T ham_ao C
@@ -853,9 +853,9 @@ int build_pairs(flosic_ctx *c) {
     c->nchunks_bf16 = (int)chunks16.size();
     if (c->nchunks_bf16 > 0) chunks16.back().flush = 1;
     c->rgc_bf16[0] = 0;
-    for (int i = 1, k = 0; i < 5; ++i) {  // run i ends after the first flush at or beyond i quarters of the rows
-        while (k < c->nchunks_bf16 && (k == 0 || !chunks16[k - 1].flush || chunks16[k].prow0 < c->rows_padded_bf16 * i / 4)) ++k;
-        c->rgc_bf16[i] = i == 4 ? c->nchunks_bf16 : k;
+    for (int i = 1, k = 0; i <= kRunsBf16; ++i) {  // run i ends after the first flush at or beyond its share of the rows
+        while (k < c->nchunks_bf16 && (k == 0 || !chunks16[k - 1].flush || chunks16[k].prow0 < c->rows_padded_bf16 * i / kRunsBf16)) ++k;
+        c->rgc_bf16[i] = i == kRunsBf16 ? c->nchunks_bf16 : k;
     }
     // segment offsets: segL[L] = first group with lA+lB >= L
     for (int L = 0; L <= 5; ++L) {
@@ -1088,7 +1088,7 @@ CoulJob<T> coulomb_job(const flosic_ctx *c, int nfb) {
     J.chunks = c->d_chunks_bf16.p;
     J.nchunks = c->nchunks_bf16;
     J.seg = c->segL;
-    for (int i = 0; i < 5; ++i) J.rgc[i] = c->rgc_bf16[i];
+    for (int i = 0; i <= kRunsBf16; ++i) J.rgc[i] = c->rgc_bf16[i];
     J.pP = c->d_pairP.p;
     J.H = form == COUL_BF16 ? (const void *)c->d_Hs.p : form == COUL_FP32 ? (const void *)c->d_H32.p
                                                                            : (const void *)c->d_H64.p;

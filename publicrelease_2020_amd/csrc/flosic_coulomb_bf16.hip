@@ -15,8 +15,8 @@ namespace flosic {
 // accumulators and 48 FP64 sums), and its H operands come from L1/L2 straight into registers.
 //
 // Split.  Block = 8 wavefronts, one block per CU (256 registers per lane).
-//   up to  48 FLOs  CW = 1: two tiles of 64 points; the four waves of a tile hold all its columns, make R and the split
-//                   by themselves for four runs of chunks, and meet in the final sum.  No barrier in the loop.
+//   up to  48 FLOs  CW = 1: two tiles of 64 points (small meshes: one); the four (eight) waves of a tile hold all its columns,
+//                   make R and the split by themselves for as many runs of chunks, and meet in the final sum.  No barrier.
 //   up to  96 FLOs  CW = 2: two tiles of 64 points; up to 192 FLOs CW = 4: one tile.  More FLOs: further blocks.
 // With CW > 1 the waves have roles, because the sums leave no room for both R and H operands loaded ahead (waves that did
 // everything in turn ran 192 FLOs, 5.2e5 rows, 2.0e5 points at 272 ms, the registers spilling, against 192 ms with roles):
@@ -29,7 +29,7 @@ namespace flosic {
 // The FP32 accumulators go into the FP64 sums at the chunks marked flush (every 256 or more rows), so the sums do not
 // depend on the split.
 // Measured, three pieces, against 16-wave blocks in which two waves of every block staged H through LDS: 10 FLOs (289 groups,
-// 3.4e4 points) 0.279 -> 0.125 ms; 30 FLOs (1686, 1.2e5) 2.98 -> 1.18; 48 FLOs (4163, 1.9e5) 12.6 -> 5.1; 64 FLOs (7371,
+// 3.4e4 points) 0.279 -> 0.097 ms; 30 FLOs (1686, 1.2e5) 2.98 -> 1.18; 48 FLOs (4163, 1.9e5) 12.6 -> 5.1; 64 FLOs (7371,
 // 2.4e5) 25.8 -> 17.5; 96 FLOs (15750, 3.7e5) 96.0 -> 68.2; 120 FLOs (24241, 3.1e5) 104 -> 85.5; 192 FLOs (60795, 2.0e5)
 // 242 -> 192.  With CW = 1 making R bounds the loop (32 and 48 FLOs take nearly the same time per row and point).  With
 // CW = 4 the MFMAs are 57% busy: of the 192 ms the MFMAs alone need 111, with A from LDS 118, with the FP64 sums 130, with
@@ -396,12 +396,11 @@ __device__ __forceinline__ void role_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// Epilogue: one column tile of sums at a time through LDS, [column][66 points]: 512 contiguous bytes per store.  With
-// CW = 1 the four row groups of a tile are added there and each stores four columns.
-template <int NP, int CW, int NT>
+// Epilogue: one column tile of sums at a time through LDS, [column][66 points]: 512 contiguous bytes per store.  The sums of
+// the RW runs of a tile (CW = 1) are added there and each stores 16 / RW columns.
+template <int NP, int RW, int NT>
 __device__ __forceinline__ void bf_store(unsigned char *__restrict__ lds, const CoulJob<__bf16> &J, const BfAcc<NP, NT> &A,
                                          int64_t kl, bool valid, int wave, int ct0, int ntmax) {
-    constexpr int RW = CW == 1 ? 4 : 1;
     const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15, rg = wave % RW, w0 = wave - rg;
     double *o = reinterpret_cast<double *>(lds);
 #pragma unroll
@@ -448,16 +447,16 @@ __device__ __forceinline__ const unsigned *bf_far_row(const CoulJob<__bf16> &J, 
     return J.far && tile * 64 < J.M ? J.far + tile * J.farw : nullptr;
 }
 
-// CW = 1: a wave on its own run of chunks, all columns
-template <int NP, int NT>
+// CW = 1: a wave on its own run of chunks (of RW), all columns
+template <int NP, int NT, int RW>
 __device__ __forceinline__ void bf_alone(unsigned char *__restrict__ lds, const CoulJob<__bf16> &J,
                                          const double *__restrict__ tab, int64_t tile, int wave, int ct0) {
-    const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15, rg = wave % 4;
+    const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15, rg = wave % RW;
     const BfPoint P = bf_point(J, tile);
     const float *ctab = (const float *)(tab + kBoysRows * kBoysCols);
     const char *zero = (const char *)(tab + kBoysTableDoubles) + lane * 16;
     float *R = reinterpret_cast<float *>(lds) + wave * bf_rsize<true>;
-    const int c0 = J.rgc[rg], c1 = J.rgc[rg + 1];
+    const int c0 = J.rgc[rg * (kRunsBf16 / RW)], c1 = J.rgc[(rg + 1) * (kRunsBf16 / RW)];
     const unsigned *far = bf_far_row(J, tile);
     // rows of a chunk beyond its groups are never written and meet zero rows of H: they only have to be finite
     for (int i = lane; i < bf_rsize<true> / 4; i += 64) ((v4f *)R)[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -499,7 +498,7 @@ __device__ __forceinline__ void bf_alone(unsigned char *__restrict__ lds, const 
         } while (!flush);
         A.flush();
     }
-    bf_store<NP, 1, NT>(lds, J, A, P.k, P.valid, wave, ct0, NT);
+    bf_store<NP, RW, NT>(lds, J, A, P.k, P.valid, wave, ct0, NT);
 }
 
 template <int NP, int CW>
@@ -642,9 +641,17 @@ __device__ __forceinline__ void bf_consumer(unsigned char *__restrict__ lds, BfT
         } while (!flush);
         A.flush();
     }
-    bf_store<NP, CW, NT>(lds, J, A, kl, kl < J.M, wave, ct0, ntmax);
+    bf_store<NP, 1, NT>(lds, J, A, kl, kl < J.M, wave, ct0, ntmax);
 }
 
+// Waves per tile with CW = 1.  Two tiles of four waves share the H that they read at the same time, one tile of eight leaves
+// less of the chip idle in the last round of 256 blocks: 48 FLOs, 2903 tiles 5.07 and 5.64 ms; 30 FLOs, 1816 tiles 1.18 and
+// 1.24; 10 FLOs, 530 tiles 0.125 and 0.097.  So eight where that saves more than a tenth of the rounds (a round of two tiles
+// counts twice).
+__host__ __device__ inline int bf_runs(int64_t M) {
+    const int64_t tiles = (M + 63) / 64;
+    return 11 * ((tiles + 255) / 256) < 20 * ((tiles + 511) / 512) ? 8 : 4;
+}
 // Work item `item` of a system: 64-point tiles 2 item and 2 item + 1 (CW = 4: tile item), column block cb of ncb; the
 // column tiles are shared out evenly over the blocks and over a block's column waves
 template <int NP, int CW, int NTLO, int NTHI>
@@ -653,15 +660,19 @@ __device__ __forceinline__ void coulomb_tile_bf16(unsigned char *__restrict__ ld
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tb0 = J.nct * cb / J.ncb, tb = J.nct * (cb + 1) / J.ncb - tb0;
     if constexpr (CW == 1) {
-        const int64_t tile = 2 * item + wave / 4;
+        const bool one = bf_runs(J.M) == 8;  // one tile per block
+        const int64_t tile = one ? item : 2 * item + wave / 4;
         if constexpr (NTHI >= 3) {
-            if (tb == 3) return bf_alone<NP, 3>(lds, J, tab, tile, wave, tb0);
+            if (tb == 3)
+                return one ? bf_alone<NP, 3, 8>(lds, J, tab, tile, wave, tb0) : bf_alone<NP, 3, 4>(lds, J, tab, tile, wave, tb0);
         }
         if constexpr (NTLO <= 2 && NTHI >= 2) {
-            if (tb == 2) return bf_alone<NP, 2>(lds, J, tab, tile, wave, tb0);
+            if (tb == 2)
+                return one ? bf_alone<NP, 2, 8>(lds, J, tab, tile, wave, tb0) : bf_alone<NP, 2, 4>(lds, J, tab, tile, wave, tb0);
         }
         if constexpr (NTLO <= 1) {
-            if (tb == 1) return bf_alone<NP, 1>(lds, J, tab, tile, wave, tb0);
+            if (tb == 1)
+                return one ? bf_alone<NP, 1, 8>(lds, J, tab, tile, wave, tb0) : bf_alone<NP, 1, 4>(lds, J, tab, tile, wave, tb0);
         }
     } else {
         const int w = wave & 3, cw = w % CW, ntmax = (tb + CW - 1) / CW;
@@ -696,7 +707,8 @@ __host__ __device__ inline int bf_col_waves(int nct, int ncb) {
 }
 int64_t bf16_items(int64_t M, int nct, int ncb) {
     const int64_t tiles = (M + 63) / 64;
-    return bf_col_waves(nct, ncb) == 4 ? tiles : (tiles + 1) / 2;
+    const int cw = bf_col_waves(nct, ncb);
+    return cw == 2 || (cw == 1 && bf_runs(M) == 4) ? (tiles + 1) / 2 : tiles;
 }
 
 template <int NP, int CW, int NTM>

@@ -54,6 +54,7 @@ struct ChunkDev {
 // the K=64 workload every 64, 128, 256, 512 rows gave |dE| against FP64 of 4.9e-7, 5.3e-7, 4.4e-7 and 6.2e-7 Ha; the
 // flush is 96 VALU instructions per wave.
 constexpr int kFlushRowsBf16 = 256;
+constexpr int kRunsBf16 = 8;
 
 // the groups by order: those of order L are [g[L], g[L + 1])
 struct FpSegs {
@@ -83,7 +84,8 @@ struct CoulJob {
     const unsigned *far;
     int farw;
     FpSegs seg;
-    int rgc[5];  // split-BF16: four runs of chunks [rgc[i], rgc[i + 1]) of about equal length that begin after a flush
+    // split-BF16: kRunsBf16 runs of chunks [rgc[i], rgc[i + 1]) of about equal length that begin after a flush
+    int rgc[kRunsBf16 + 1];
 };
 
 // Column-block widths that may be asked for: nfb must divide ldh (nF rounded up to a multiple of coulomb_cols); the

@@ -48,3 +48,31 @@ def test_tile_edges(K, up, dn, nrad, nang, box, monkeypatch):
     print(f"{up + dn} FLOs, {sysm.mesh.npts} points: three pieces {d3:.1e}, two {d2:.1e}", flush=True)
     assert d3 <= 1e-5
     assert d2 <= 3e-3
+
+
+@pytest.mark.parametrize("M", [256 * 64, 256 * 64 + 1, 512 * 64, 512 * 64 + 1, 768 * 64 + 1])
+def test_waves_per_tile(M, monkeypatch):
+    """Mesh sizes on both sides of the limits between eight waves on one tile and four on each of two (up to 48 FLOs): 256 and
+    512 tiles; the tolerance as above, and the batched launch gives the same bits."""
+    import dataclasses
+    from publicrelease_2020_amd import flosic as F
+    full = S.make_synthetic(2, 9, 61, S.XC_LSDA, nrad=150, nang=194, box=5.0)
+    idx = np.arange(M) % full.mesh.npts
+    sysm = dataclasses.replace(full, mesh=S.Mesh(xyz=np.ascontiguousarray(full.mesh.xyz[idx]),
+                                                 w=np.ascontiguousarray(full.mesh.w[idx])))
+    e = F.Flosic(0)
+    e.load_system(sysm, 2)
+    e.evaluate()
+    got = _vh(e, sysm)
+    b = F.FlosicBatch([e])
+    b.evaluate()
+    assert np.array_equal(_vh(e, sysm), got)
+    b.close()
+    e.close()
+    monkeypatch.setenv("FLOSIC_COULOMB", "valu")
+    e = F.Flosic(0)
+    e.load_system(sysm, 0)
+    e.evaluate()
+    ref = _vh(e, sysm)
+    e.close()
+    assert np.abs(got - ref).max() <= 1e-5 * np.abs(ref).max()
