@@ -191,10 +191,11 @@ void launch_prim_coef(int nps, const int *ps_f0, const int *ps_stride, const int
 // recursion; H[row+tuv][f] = sym * 2pi/p * sum_{mu,nu} dA[mu][f] dB[nu][f] Ex Ey Ez
 //
 // Bound: latency, a few microseconds of work per block at any system size.  One block per group: 27 threads raise the
-// E^{ij}_t of one axis and (i, j) in registers; the products Ex Ey Ez of every (component pair, tuv) go to LDS, wave = pair,
-// lane = tuv; then a thread holds one (tuv, FLO) and runs over the component pairs, up to 100, from LDS.  A thread that held all
-// 35 sums of one FLO (indexed at run time, so in scratch memory) left 54 of 64 lanes idle at 10 FLOs and took 190 us
-// there (289 groups), 229 at 30 FLOs (1686 groups), 525 at 96 FLOs (15750); now 27, 82 and 279.
+// E^{ij}_t of one axis and (i, j) in registers; the products Ex Ey Ez of every (component pair, tuv) go to LDS, wave = component
+// of the first centre, lane = tuv; then a thread holds one (tuv, FLO) and runs over the component pairs, up to 100, from LDS,
+// five loads at a time.  A thread that held all 35 sums of one FLO (indexed at run time, so in scratch memory) left 54 of
+// 64 lanes idle at 10 FLOs and took 190 us there (289 groups), 229 at 30 FLOs (1686 groups), 525 at 96 FLOs (15750); with one
+// load after the other and the pairs one by one over the waves 27, 82 and 279; now 17, 60 and 262.
 // ---------------------------------------------------------------------------------------------------
 constexpr int kHermThreads = 256, kHermCols = 64;
 __device__ __forceinline__ void e_raise(double (&v)[5], double shift, double inv2p) {
@@ -215,7 +216,7 @@ __global__ void __launch_bounds__(kHermThreads) k_hermite(const PairDev *__restr
     __shared__ double E[3][3][3][5], C[100 * 35], dA[10][kHermCols], dB[10][kHermCols];
     const PairDev pr = pairs[blockIdx.x];
     const double p = pr.a + pr.b;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (tid < 27) {
         const int d = tid / 9, i = tid / 3 % 3, j = tid % 3;
         const double A = d == 0 ? pr.A[0] : d == 1 ? pr.A[1] : pr.A[2], B = d == 0 ? pr.B[0] : d == 1 ? pr.B[1] : pr.B[2];
@@ -244,13 +245,13 @@ __global__ void __launch_bounds__(kHermThreads) k_hermite(const PairDev *__restr
         const int pos = min(lane, 34) - ord * (ord + 1) * (ord + 2) / 6;
         const int uv = pos < 1 ? 0 : pos < 3 ? 1 : pos < 6 ? 2 : pos < 10 ? 3 : 4;
         const int t = ord - uv, v = pos - uv * (uv + 1) / 2, u = uv - v;
-        int e = 0;
-        for (int ma = mA; ma; ma &= ma - 1) {
+        for (int ma = mA, ia = 0; ma; ma &= ma - 1, ++ia) {
+            if ((ia & 3) != wave) continue;
             const int a = __builtin_ctz(ma), ax = cpow(a, 0), ay = cpow(a, 1), az = cpow(a, 2);
-            for (int mb = mB; mb; mb &= mb - 1, ++e) {
-                if ((e & 3) != wave) continue;
+            double *c = C + ia * nB * nt + lane;
+            for (int mb = mB; mb; mb &= mb - 1, c += nt) {
                 const int b = __builtin_ctz(mb), bx = cpow(b, 0), by = cpow(b, 1), bz = cpow(b, 2);
-                if (lane < nt) C[e * nt + lane] = E[0][ax][bx][t] * E[1][ay][by][u] * E[2][az][bz][v];
+                if (lane < nt) *c = E[0][ax][bx][t] * E[1][ay][by][u] * E[2][az][bz][v];
             }
         }
     }
@@ -276,7 +277,18 @@ __global__ void __launch_bounds__(kHermThreads) k_hermite(const PairDev *__restr
             double h = 0.0;
             for (int m = 0; m < nA; ++m) {
                 const double da = dA[m][fl];
-                for (int n = 0; n < nB; ++n, c += nt) h += da * dB[n][fl] * *c;
+                int n = 0;
+                for (; n + 5 <= nB; n += 5, c += 5 * nt) {  // ten of an spd centre: the LDS loads of five go out together
+                    double b[5], x[5];
+#pragma unroll
+                    for (int e = 0; e < 5; ++e) {
+                        b[e] = dB[n + e][fl];
+                        x[e] = c[e * nt];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 5; ++e) h += da * b[e] * x[e];
+                }
+                for (; n < nB; ++n, c += nt) h += da * dB[n][fl] * *c;
             }
             H[(int64_t)(pr.row + tuv) * ldh + f0 + fl] = fac * h;
         }
