@@ -701,7 +701,7 @@ __device__ __forceinline__ void coulomb_tile_bf16(unsigned char *__restrict__ ld
     }
 }
 
-__host__ __device__ inline int bf_col_waves(int nct, int ncb) {
+__host__ __device__ constexpr int bf_col_waves(int nct, int ncb) {
     const int tb = (nct + ncb - 1) / ncb;
     return tb <= 3 ? 1 : tb <= 6 ? 2 : 4;
 }
@@ -714,6 +714,7 @@ int64_t bf16_items(int64_t M, int nct, int ncb) {
 template <int NP, int CW, int NTM>
 __global__ void __launch_bounds__(512, 2) k_coulomb_bf16(CoulJob<__bf16> J, const double *__restrict__ tab) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[bf_lds<NP, CW>];
+    static_assert(split_covered(bf_col_waves, 192, CW, (NTM > 1 ? NTM - 1 : 1), NTM, true), "a wave's tiles have no instance");
     coulomb_tile_bf16<NP, CW, (NTM > 1 ? NTM - 1 : 1), NTM>(lds, J, tab, blockIdx.x, blockIdx.y);
 }
 
@@ -727,9 +728,12 @@ __global__ void __launch_bounds__(512, 2) k_coulomb_bf16_batch_all(const CoulJob
     const CoulJob<__bf16> J = uniform_job(jobs, j);
     const int64_t item = local / J.ncb;
     const int cb = (int)(local - item * J.ncb);
+    static_assert(split_covered(bf_col_waves, 192, 1, 1, 3, false) && split_covered(bf_col_waves, 192, 2, 1, 3, false) &&
+                      split_covered(bf_col_waves, 192, 4, 1, 3, false), "a wave's tiles have no instance");
     switch (bf_col_waves(J.nct, J.ncb)) {
         case 1: coulomb_tile_bf16<NP, 1, 1, 3>(lds, J, tab, item, cb); break;
-        case 2: coulomb_tile_bf16<NP, 2, 2, 3>(lds, J, tab, item, cb); break;
+        // blocks of 64 columns share 7, 10, 11 .. tiles out as three and four: the waves of three hold one and two
+        case 2: coulomb_tile_bf16<NP, 2, 1, 3>(lds, J, tab, item, cb); break;
         default: coulomb_tile_bf16<NP, 4, 1, 3>(lds, J, tab, item, cb); break;
     }
 }

@@ -58,7 +58,7 @@ inline int fp_units(const FpSegs &s) {
     return n;
 }
 // column waves of a block
-__host__ __device__ inline int fp_col_waves(int nct, int ncb) {
+__host__ __device__ constexpr int fp_col_waves(int nct, int ncb) {
     const int tb = (nct + ncb - 1) / ncb;
     return tb <= 4 ? 1 : tb <= 6 ? 2 : 4;
 }
@@ -300,6 +300,7 @@ constexpr int fp_waves_per_simd = NTM > 2 || (CW > 1 && sizeof(T) == 8) ? 2 : 5 
 template <typename T, int CW, int NTM>
 __global__ void __launch_bounds__(256, (fp_waves_per_simd<T, CW, NTM>)) k_coulomb_fp(CoulJob<T> J, const double *__restrict__ tab) {
     __shared__ FpTileLds<T> lds;
+    static_assert(split_covered(fp_col_waves, 256, CW, (NTM > 1 ? NTM - 1 : 1), NTM, true), "a wave's tiles have no instance");
     coulomb_tile_fp<T, CW, (NTM > 1 ? NTM - 1 : 1), NTM>(lds, J, tab, blockIdx.x, blockIdx.y);
 }
 
@@ -313,6 +314,8 @@ __global__ void __launch_bounds__(256, 2) k_coulomb_fp_batch_all(const CoulJob<T
     const CoulJob<T> J = uniform_job(jobs, j);
     const int64_t tile = local / J.ncb;
     const int cb = (int)(local - tile * J.ncb);
+    static_assert(split_covered(fp_col_waves, 256, 1, 1, 4, false) && split_covered(fp_col_waves, 256, 2, 2, 3, false) &&
+                      split_covered(fp_col_waves, 256, 4, 1, 3, false), "a wave's tiles have no instance");
     switch (fp_col_waves(J.nct, J.ncb)) {
         case 1: coulomb_tile_fp<T, 1, 1, 4>(lds, J, tab, tile, cb); break;
         case 2: coulomb_tile_fp<T, 2, 2, 3>(lds, J, tab, tile, cb); break;

@@ -4,10 +4,6 @@
 namespace flosic {
 
 int64_t fp_steps(const FpSegs &seg) { return seg_step0(seg, 5); }
-int coulomb_col_blocks(int nF, int nfb) {
-    const int tb = std::min(nfb / 16, 12);  // column tiles of a block
-    return std::max(1, ((nF + 15) / 16 + tb - 1) / tb);
-}
 
 template void launch_frag_h<double>(const FpSegs &, const double *, int, int, double *, hipStream_t);
 template void launch_coulomb_mfma<double>(const FpSegs &, const double4 *, const double *, const double *, const double *,

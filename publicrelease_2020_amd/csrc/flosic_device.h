@@ -281,6 +281,29 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t v) {
     const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((uint64_t)v >> 32));
     return (int64_t)(((uint64_t)hi << 32) | lo);
 }
+// Column tiles that a launch shares out: block cb of ncb takes tiles nct cb / ncb to nct (cb + 1) / ncb - 1, column wave cw of
+// its CW likewise.  A wave whose count has no compiled instance would return with its columns unwritten, so every kernel
+// asserts that its instances, those of NTLO to NTHI tiles, cover every share-out (cws(nct, ncb) the column waves of a block;
+// blocks of the legal widths up to `widest` columns; 128 tiles are 2048 FLOs, and the counts per wave recur long before).
+// single: the instances of the launch for one system, built for its largest wave's tiles and one less.
+template <typename F>
+constexpr bool split_covered(F cws, int widest, int CW, int NTLO, int NTHI, bool single) {
+    for (int nfb = 64; nfb <= widest; nfb += 64)
+        for (int nct = 1; nct <= 128; ++nct) {
+            const int ncb = coulomb_col_blocks(16 * nct, nfb);
+            if (cws(nct, ncb) != CW) continue;
+            const int ntm = ((nct + ncb - 1) / ncb + CW - 1) / CW;
+            if (single && ntm != NTHI) continue;
+            for (int cb = 0; cb < ncb; ++cb) {
+                const int tb = nct * (cb + 1) / ncb - nct * cb / ncb;
+                for (int cw = 0; cw < CW; ++cw) {
+                    const int nt = tb * (cw + 1) / CW - tb * cw / CW;
+                    if (nt < NTLO || nt > NTHI) return false;
+                }
+            }
+        }
+    return true;
+}
 // block -> (job, local item): off[] ascending, off[0] = 0
 __device__ __forceinline__ int job_of_block(const int64_t *__restrict__ off, int njobs, int64_t it, int64_t &local) {
     int lo = 0, hi = njobs - 1;  // largest j with off[j] <= it

@@ -129,7 +129,11 @@ void launch_coulomb(const int *segL /*6 offsets*/, const double4 *pairP, const i
 // kernels then generate R_tuv of every (point, group) and stream H.  T = double (FP64 MFMA) or float (FP32 MFMA, FP64
 // sums per chunk of <= 64 rows): fp_steps K steps of 4 rows, at most nfb FLO columns per block.
 int64_t fp_steps(const FpSegs &seg);
-int coulomb_col_blocks(int nF, int nfb);
+// column blocks of a launch: as few of at most nfb columns (and 12 tiles of 16) as hold all FLOs
+constexpr int coulomb_col_blocks(int nF, int nfb) {
+    const int tb = nfb / 16 < 12 ? nfb / 16 : 12, n = ((nF + 15) / 16 + tb - 1) / tb;
+    return n > 1 ? n : 1;
+}
 template <typename T>
 void launch_frag_h(const FpSegs &seg, const double *H, int ldh, int nF, T *Hf, hipStream_t s);
 template <typename T>
