@@ -1050,15 +1050,40 @@ void launch_gather(const double *src, int64_t stride, int n, double *dst, hipStr
 }
 
 // Deterministic compensated (Neumaier) reduction of per-block partials, out[f][q] = sum_b partial[f][b][q]; with accumulate
-// the sum starts from out.  Bound: the latency of the loads, so 16 waves share the partials of 64 outputs (consecutive
+// the sum starts from out.  Two shapes:
+// k_reduce_partials, few outputs: bound by the latency of the loads, so 16 waves share the partials of 64 outputs (consecutive
 // ranges of b, eight loads in flight) and their sums are added in order, compensated again.  One thread per output, one
 // load after the other, took 22 us at 90 outputs of 132 partials (10 FLOs, 3.4e4 points), 62 at 30 FLOs (1.2e5 points) and
 // 188 at 96 FLOs (3.7e5 points), each an average over the sums of a pass; now 4.2, 6.0 and 14.7.
+// k_reduce_many, many outputs (those of V^i_ab, n^3, and of the products over a block of the mesh, with few partials each):
+// bound by memory, a thread per output, four loads in flight, no LDS.  16 waves per 64 outputs, most of them without a
+// partial, took 117 us at 1.7e6 outputs (n = 120) of 8 partials, here 25 (5.5 TB/s); at 1e6 of 2 57 and 5.6.
+// The limit (us, 16 waves and one thread): 2 partials of 1.6e4 outputs 2.8 and 2.7, of 6.4e4 5.2 and 2.4; 8 of 1.6e4 3.0 and
+// 2.7, of 6.4e4 5.4 and 3.6; 32 of 6.4e4 6.5 and 6.7, of 2.5e5 26 and 13; 128 of 6.4e4 14 and 27, of 2.5e5 48 and 43; 1024
+// of 1.6e4 25 and 180, of 2.5e5 336 and 325: one thread from 2048 outputs per partial or 2^17 outputs on.
 constexpr int kRedWaves = 16;
 __device__ __forceinline__ void neumaier(double x, double &s, double &c) {
     const double t = s + x;
     c += fabs(s) >= fabs(x) ? (s - t) + x : (x - t) + s;
     s = t;
+}
+__global__ void __launch_bounds__(256) k_reduce_many(const double *__restrict__ partial, int n, int nblk, int nq,
+                                                     double *__restrict__ out, int accumulate) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int f = i / nq;
+    const double *p = partial + (int64_t)f * nblk * nq + i - f * nq;
+    double s = accumulate ? out[i] : 0.0, c = 0.0;
+    for (int b = 0; b < nblk; b += 4, p += (int64_t)4 * nq) {
+        double x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (b + j < nblk) x[j] = p[(int64_t)j * nq];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (b + j < nblk) neumaier(x[j], s, c);
+    }
+    out[i] = s + c;
 }
 __global__ void __launch_bounds__(64 * kRedWaves) k_reduce_partials(const double *__restrict__ partial, int n, int nblk,
                                                                     int nq, double *__restrict__ out, int accumulate) {
@@ -1099,6 +1124,11 @@ void launch_reduce_partials(const double *partial, int nF, int nblk, int nq, dou
                             bool accumulate) {
     const int n = nF * nq;
     if (n <= 0) return;
+    if (n >= std::min<int64_t>(1 << 17, (int64_t)2048 * nblk)) {
+        hipLaunchKernelGGL(k_reduce_many, dim3((unsigned)(((int64_t)n + 255) / 256)), dim3(256), 0, s, partial, n, nblk, nq, out,
+                           accumulate ? 1 : 0);
+        return;
+    }
     hipLaunchKernelGGL(k_reduce_partials, dim3((n + 63) / 64), dim3(64 * kRedWaves), 0, s, partial, n, nblk, nq, out,
                        accumulate ? 1 : 0);
 }
