@@ -1019,10 +1019,7 @@ int gemm_tn_points(flosic_ctx *c, int rows, int n, const double *A, const double
     if (lda <= 0) lda = M;
     if (ldb <= 0) ldb = M;
     int nparts;
-    if (rows >= 512 && n > 80 && nplane == 1) {
-        // large in all three dimensions: the library's LDS-tiled product, batched over 64 point slices (1720 x 192 and
-        // 368 437 points: 4.1 ms against 6.0; 916 x 96, 370 513: 1.46 against 1.70; even at 792 x 72, and 128 x 20 with
-        // 69 773 points takes it 0.24 against 0.06, because two dimensions fill too few of its 128 x 64 tiles)
+    if (nplane == 1 && tn_by_library(rows, n, M)) {  // batched over point slices
         const double one = 1.0, zero = 0.0;
         int nsl = 64;
         while (nsl > 1 && M / nsl < 4096) --nsl;
@@ -2160,10 +2157,12 @@ int32_t flosic_siclag_der(flosic_ctx *c, double *dersic) {
     const int64_t M = c->M;
     const bool blocked = c->block_pts > 0;
     ALLOC(c, c->d_dG, (size_t)3 * N * nF);
-    // The planes lie one behind the other: one product of 3 N rows up to 80 FLOs (48 FLOs, N = 458, 32 768 points: 145 us
-    // against 3 x 67).  Beyond, products are large enough one by one, and the stacked one is no faster (192 FLOs,
-    // N = 1832: 1.78 ms against 3 x 0.46).
-    const bool stacked = nF <= 80;
+    const int64_t mb = !blocked && nd == 10 ? M : blocked ? mesh_block(c) : std::min<int64_t>(M, kDerBlockPts);
+    // The planes lie one behind the other: one product of 3 N rows where k_tn takes it (48 FLOs, N = 604, 32 768 points:
+    // 147 us against 3 x 61; 96 FLOs 247 against 3 x 97; 32 FLOs and N = 388 82 against 3 x 38).  Products beyond that
+    // are large enough one by one, and the library is slower on the stacked planes (128 FLOs, N = 1832: 915 us against
+    // 3 x 262; 192 FLOs 1800 against 3 x 505).
+    const bool stacked = !tn_by_library(3 * N, nF, mb);
     auto products = [&](const double *A, const double *u, int64_t m, int64_t ldu, bool accumulate) -> int {
         if (stacked) return gemm_tn_points(c, 3 * N, nF, A, u, m, c->d_dG.p, accumulate, m, ldu);
         for (int d = 0; d < 3; ++d) {
@@ -2175,7 +2174,6 @@ int32_t flosic_siclag_der(flosic_ctx *c, double *dersic) {
     if (!blocked && nd == 10) {  // resident PBE planes: value, gradient, Hessian of every function on the mesh
         if ((r = products(c->d_planes.p + (size_t)N * M, c->d_U.p, M, M, false))) return r;
     } else {
-        const int64_t mb = blocked ? mesh_block(c) : std::min<int64_t>(M, kDerBlockPts);
         const int nblk = (int)((M + 255) / 256);
         // mesh-block mode needs the value planes too (the FLO fields are rebuilt); resident LSDA only the gradients
         const int pk = blocked ? ng : -3, np = blocked ? ng : 3, g0 = blocked ? 1 : 0;

@@ -147,8 +147,8 @@ void launch_orbitals(const double *planes, int64_t m, int nd, int N, const doubl
 // Bound: 2 rows n M / 77 TFLOP/s or 8 (rows + n) M bytes.  Blocks go to the 8 XCDs round robin, and a slice's tiles (which
 // read the same points) are numbered 8 apart: they meet in one XCD's L2.  Measured with the final sum, against the
 // library's product batched over point slices of at least 4096: 12 x 10, 11 640 points 320 -> 19 us; 128 x 20, 69 773
-// 236 -> 58 us; 260 x 30 and four 15 x 15 planes per spin, 116 200 2.12 -> 0.45 ms; equal at 500 x 48 (0.27 -> 0.29 ms)
-// and 792 x 72.
+// 236 -> 58 us; 260 x 30 and four 15 x 15 planes per spin, 116 200 2.12 -> 0.45 ms; equal at 500 x 48 (0.27 -> 0.29 ms).
+// Which of the two takes a product: tn_by_library.
 // ---------------------------------------------------------------------------------------------------
 // k: the first of this lane's points (2 lr into the block)
 template <int NT, bool TAIL>
@@ -279,6 +279,21 @@ TnPlan tn_plan(int rows, int n, int64_t M, int nplane) {
     return p;
 }
 }  // namespace
+
+// The library's LDS-tiled product (batched over point slices) computes whole multiples of 64 columns, k_tn whole multiples of a
+// wave's, reading A once for each.  Small products give the library too few tiles: about 230 us at any size.  Library and
+// k_tn in us, work in rows x columns x points: 604 x 64, 32768 points (1.3e9) 230 and 78, 65536 (2.5e9) 236 and 139, 370001
+// (1.4e10) 664 and 910; 604 x 128, 32768 (2.5e9) 227 and 127, 65536 (5.1e9) 238 and 236; 1208 x 128, 32768 (5.1e9) 235 and
+// 234, 120001 (1.9e10) 723 and 816; 1832 x 192, 370001 4266 and 6456: from 5e9 on.  Above 192 columns tall products gain
+// earlier: 1208 x 224, 8192 (2.2e9) 231 and 129, 1832 x 224 (3.4e9) 146 and 172, 1832 x 256 (3.8e9) 145 and 201: from 3e9 on.
+// Where k_tn pads less (65 to 96 and 129 to 144 columns) it holds out longer: 604 x 96, 120001 (7e9) 474 and 341; 604 x 144,
+// 370001 (3.2e10) 1473 and 1243; 1832 x 96, 120001 (2.1e10) 933 and 1075, 370001 (6.5e10) 2758 and 3173: from 3e10 on.
+bool tn_by_library(int rows, int n, int64_t M) {
+    if (n <= 48) return false;  // one column group: 604 x 48, 370001 points 608 and 587 us
+    const TnPlan p = tn_plan(rows, n, M, 1);
+    const bool pads_less = 16 * p.cb * p.cg < (n + 63) / 64 * 64;
+    return (double)rows * n * (double)M >= (n > 192 ? 3e9 : pads_less ? 3e10 : 5e9);
+}
 
 int tn_slices(int rows, int n, int64_t M, int nplane) { return tn_plan(rows, n, M, nplane).nsl * nplane; }
 

@@ -172,6 +172,7 @@ void launch_orbitals(const double *planes, int64_t m, int nd, int N, const doubl
 // part[slice][r + rows c], tn_slices(...) slices in all, whose sum is sum_p sum_k A[p sa + k + lda r] B[p sb + k + ldb c]
 // over nplane planes and M points
 int tn_slices(int rows, int n, int64_t M, int nplane);
+bool tn_by_library(int rows, int n, int64_t M);  // the library's product is the faster one
 void launch_tn(const double *A, int64_t lda, int64_t sa, const double *B, int64_t ldb, int64_t sb, int rows, int n,
                int64_t M, int nplane, double *part, hipStream_t s);
 
