@@ -121,13 +121,19 @@ struct DevBuf {
 struct PinBuf {
     double *p = nullptr;
     size_t n = 0;
+    bool busy = false;  // copies from or to it have been queued and not been waited for
     ~PinBuf() {
         if (p) (void)hipHostFree(p);
     }
-    // at least cnt doubles; the contents are lost when it grows, and copies on s that still use it are waited for
+    // at least cnt doubles, free to be written: copies on s that still use it are waited for; the contents are lost when it
+    // grows
     bool ensure(size_t cnt, hipStream_t s) {
+        if (busy || (p && cnt > n)) {
+            if (hipStreamSynchronize(s) != hipSuccess) return false;
+            busy = false;
+        }
         if (cnt <= n) return true;
-        if (p && (hipStreamSynchronize(s) != hipSuccess || hipHostFree(p) != hipSuccess)) return false;
+        if (p && hipHostFree(p) != hipSuccess) return false;
         p = nullptr;
         n = 0;
         if (hipHostMalloc((void **)&p, cnt * sizeof(double), hipHostMallocDefault) != hipSuccess) {
@@ -953,8 +959,8 @@ int run_frmorb(flosic_ctx *c) {
     ALLOC(c, c->d_cflo, (size_t)N * nfod);
     // One copy brings the FOD coordinates and the KS orbitals of both spins, one takes the orbitals at the FODs back, one
     // brings both TMAT; the only wait is the one for the middle one.  (Eight copies out of and into ordinary memory, each
-    // waiting for the stream, made this stage 0.2 ms of host time at any size.)  The staging memory is free again when
-    // it is written: every pass waits for its own orbitals at the FODs, which lie behind the copies of the pass before.
+    // waiting for the stream, made this stage 0.2 ms of host time at any size.)  The copy of TMAT is still on its way when
+    // this returns: an evaluation waits for results that lie behind it, any other caller's next pass for the stream.
     const FoLayout fo(c);
     const size_t npsi = 4 * fo.ntm;
     ALLOC(c, c->d_foin, fo.total);
@@ -968,6 +974,7 @@ int run_frmorb(flosic_ctx *c) {
         for (int d = 0; d < 3; ++d) h_in[(size_t)d * nfod + t] = f[d];
     }
     for (int s = 0; s < 2; ++s) std::copy(c->sp[s].coef.begin(), c->sp[s].coef.end(), h_in + fo.coef[s]);
+    c->h_fo.busy = true;
     HIPCHK(c, hipMemcpyAsync(c->d_foin.p, h_in, sizeof(double) * fo.total, hipMemcpyHostToDevice, c->stream));
     // chi planes [K][mu][FOD], K = value, d/dx, d/dy, d/dz
     launch_basis_planes<double>(basis_view(c), c->d_foin.p, c->d_foin.p + nfod, c->d_foin.p + 2 * nfod, nfod, 4,
@@ -986,6 +993,7 @@ int run_frmorb(flosic_ctx *c) {
     }
     HIPCHK(c, hipMemcpyAsync(h_psi, c->d_psi.p, sizeof(double) * npsi, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->h_fo.busy = false;
     int bad[2] = {0, 0};
     host_parallel(2, [&](int s0, int s1) {
         for (int s = s0; s < s1; ++s)
@@ -997,6 +1005,7 @@ int run_frmorb(flosic_ctx *c) {
                         c->sp[s].q[bad[s] - 1]);
     for (int s = 0; s < 2; ++s)
         if (c->sp[s].nocc > 0) std::copy(c->sp[s].tmat.begin(), c->sp[s].tmat.end(), h_tmat + fo.tm[s]);
+    c->h_fo.busy = true;
     HIPCHK(c, hipMemcpyAsync(c->d_tmat.p, h_tmat, sizeof(double) * fo.ntm, hipMemcpyHostToDevice, c->stream));
     for (int s = 0, off = 0; s < 2; off += c->sp[s].nocc, ++s) {
         const int n = c->sp[s].nocc;
@@ -1467,6 +1476,7 @@ int eval_finish(flosic_ctx *c) {
         if ((r = queue_results(c))) return r;
         HIPCHK(c, hipStreamSynchronize(c->stream));
     }
+    c->h_fo.busy = false;  // its copies lie before the results on the stream
     take_results(c);
     // RESULTS(1:13) per FLO (apotnl_sic.F:564-623)
     c->zsic = 0.0;
@@ -2320,7 +2330,8 @@ int32_t flosic_lagmult_slv(flosic_ctx *c, int32_t ispn, const double *pot, int32
     const int nd = xc_planes(c);
     ALLOC(c, c->d_pot, (size_t)M);
     if (!c->h_pot.ensure((size_t)M + (size_t)n * n, c->stream)) return fail(c, FLOSIC_ENOMEM, "host staging memory");
-    std::copy(pot, pot + M, c->h_pot.p);  // the previous call has waited for its result, which lies behind its copy
+    std::copy(pot, pot + M, c->h_pot.p);
+    c->h_pot.busy = true;
     HIPCHK(c, hipMemcpyAsync(c->d_pot.p, c->h_pot.p, sizeof(double) * M, hipMemcpyHostToDevice, c->stream));
     ALLOC(c, c->d_lap, (size_t)(nd == 10 ? 3 : 1) * n * mb);
     ALLOC(c, c->d_wop, (size_t)n * mb);
@@ -2360,6 +2371,7 @@ int32_t flosic_lagmult_slv(flosic_ctx *c, int32_t ispn, const double *pot, int32
     double *L = c->h_pot.p + M;
     HIPCHK(c, hipMemcpyAsync(L, c->d_small.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->h_pot.busy = false;
     for (int k = 0; k < n; ++k)
         for (int j = 0; j < n; ++j) sic[j + (size_t)ldsic * k] += L[j + (size_t)n * k];
     return FLOSIC_OK;
