@@ -1591,9 +1591,10 @@ std::vector<uint64_t> batch_sig(const flosic_batch *b) {
     return v;
 }
 
-// Classes of equal (form, pieces), each one launch whatever the members' column-block widths; jobs heaviest first
-// (work per item ~ K steps x columns), so that the longest items are dispatched first and the hardware dispatcher
-// balances the tail.  The job records and item offsets go to device memory once per plan.
+// Classes of equal (form, pieces), each one launch whatever the members' column-block widths; jobs heaviest first, so that
+// the longest items are dispatched first and the hardware dispatcher balances the tail.  Work of an item: K steps times
+// the column tiles of its block and one more, which stands for R, times its 64-point tiles.  The job records and item
+// offsets go to device memory once per plan.
 int build_plan(flosic_batch *b) {
     static_assert(sizeof(CoulJob<double>) == sizeof(CoulJob<float>) && sizeof(CoulJob<double>) == sizeof(CoulJob<__bf16>),
                   "job layout is independent of the operand type");
@@ -1619,9 +1620,15 @@ int build_plan(flosic_batch *b) {
     for (auto &k : b->classes) {
         std::vector<CoulJob<double>> jobs;
         for (int i : k.members) jobs.push_back(coulomb_job<double>(b->ctxs[i], coulomb_nfb(b->ctxs[i])));
-        std::stable_sort(jobs.begin(), jobs.end(), [](const CoulJob<double> &x, const CoulJob<double> &y) {
-            return x.nsteps * x.nfb > y.nsteps * y.nfb;
-        });
+        auto items_of = [&](const CoulJob<double> &J) {  // per column block
+            return k.form == COUL_BF16 ? bf16_items(J.M, J.nct, J.ncb) : (J.M + 63) / 64;
+        };
+        auto work = [&](const CoulJob<double> &J) {
+            const int64_t items = items_of(J);
+            return J.nsteps * ((J.nct + J.ncb - 1) / J.ncb + 1) * (((J.M + 63) / 64 + items - 1) / items);
+        };
+        std::stable_sort(jobs.begin(), jobs.end(),
+                         [&](const CoulJob<double> &x, const CoulJob<double> &y) { return work(x) > work(y); });
         k.job0 = (int64_t)all.size();
         k.off0 = (int64_t)offs.size();
         k.njobs = (int)jobs.size();
@@ -1629,7 +1636,7 @@ int build_plan(flosic_batch *b) {
         for (const auto &J : jobs) {
             all.push_back(J);
             offs.push_back(items);
-            items += (k.form == COUL_BF16 ? bf16_items(J.M, J.nct, J.ncb) : (J.M + 63) / 64) * J.ncb;
+            items += items_of(J) * J.ncb;
         }
         offs.push_back(items);
         if (items >= (int64_t)INT32_MAX)
