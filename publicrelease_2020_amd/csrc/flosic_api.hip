@@ -1148,8 +1148,8 @@ void coulomb_launch(flosic_ctx *c, const double *x, const double *y, const doubl
     }
 }
 
-// The autotuner: every legal column-block width of the context's Coulomb form is timed on a strided sample of at
-// most 32768 mesh points (every point of a small mesh) and the fastest kept.  Results are cached per process by
+// The autotuner: every legal column-block width of the context's Coulomb form that gives another launch is timed on a strided
+// sample of at most 32768 mesh points (every point of a small mesh) and the fastest kept.  Results are cached per process by
 // form, FLO count, Hermite rows and mesh size, so equal shapes are tuned once.
 std::mutex g_tune_mu;
 std::map<std::string, int> g_tune_cache;
@@ -1184,10 +1184,13 @@ int autotune_coulomb(flosic_ctx *c) {
     launch_gather(c->d_y.p, stride, (int)S, c->d_ty.p, c->stream);
     launch_gather(c->d_z.p, stride, (int)S, c->d_tz.p, c->stream);
     HIPCHK(c, hipGetLastError());
-    int best = 0;
+    int best = 0, blocks = 0;
     float best_ms = 0.f;
     for (int nfb : {256, 192, 128, 64}) {
         if (!coulomb_cols_legal(nfb, c->ldh, form == COUL_BF16)) continue;
+        // the same launch as a wider one's (200 FLOs: 256 and 128 both give two blocks)
+        if (coulomb_col_blocks(c->nF, nfb) == blocks) continue;
+        blocks = coulomb_col_blocks(c->nF, nfb);
         float ms = 0.f;
         for (int rep = 0; rep < 2; ++rep) {  // the second launch is timed
             HIPCHK(c, hipEventRecord(c->ev[EV_COUL0], c->stream));

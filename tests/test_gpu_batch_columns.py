@@ -41,3 +41,18 @@ def test_uneven_blocks(K, up, dn, prec):
     assert np.array_equal(_vh(e, sysm), ref)
     b.close()
     e.close()
+
+
+def test_autotuned_width():
+    """200 FLOs: blocks of 256 and of 128 columns are the same launch, which counts as the wider one."""
+    from publicrelease_2020_amd import flosic as F
+    sysm = S.make_synthetic(24, 100, 64, S.XC_LSDA, nrad=4, nang=26, box=8.0)
+    e = F.Flosic(0)
+    e.load_system(sysm)
+    e.evaluate()
+    ref = _vh(e, sysm)
+    e.set_coulomb_cols(-1)
+    e.evaluate()
+    assert e.coulomb_cols() in (256, 64)
+    assert np.abs(_vh(e, sysm) - ref).max() <= 1e-12 * np.abs(ref).max()  # FP64 sums of other runs of rows
+    e.close()
