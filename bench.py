@@ -69,17 +69,25 @@ def coulomb_flops(counts) -> float:
     return 2.0 * M * rows * nF
 
 
+def coulomb_bytes(counts, prec: str) -> float:
+    """Compulsory HBM bytes of one Coulomb launch: H once in the form's operands (the streamed Hermite rows, columns
+    rounded up to tiles of 16), V_H written once, the mesh coordinates."""
+    hbytes = {"fp64": 8, "mixed": 4, "bf16x3": 6, "bf16x2": 4}[prec]
+    M, nF = float(counts[2]), int(counts[4])
+    return float(counts[6]) * ((nF + 15) // 16 * 16) * hbytes + 8.0 * M * nF + 24.0 * M
+
+
 def phase_roofline(sysm, counts, phases_ms, prec_name: str) -> dict:
     """Per-phase algorithmic work of one evaluation against the bound of each phase.  nd = field planes (1 LSDA,
     10 PBE: value, gradient, Hessian), n_s = FLOs of spin s.
-      orbitals   phi = Phi_d C~ on the mesh (rocBLAS dgemm): 2 M N nF nd flops; reads the basis planes and writes
+      orbitals   phi = Phi_d C~ on the mesh (FP64 MFMA): 2 M N nF nd flops; reads the basis planes and writes
                  the FLO fields, 8 M nd (N + nF) bytes
       xc_energy  XC, V_tot, U and the energy partial sums: reads nd field planes and V_H, writes V_tot and U
                  (PBE: and 4 planes of the exact derivative), 8 M nF (nd + 3 [+ 4]) bytes
-      sic_matrix G = Phi^T U split over point slices (dgemm): 2 M N nF flops (PBE: + 4 x 2 M n_s^2 for SIC_ex),
-                 8 M (N + nF) bytes
+      sic_matrix G = Phi^T U split over point slices (FP64 MFMA, large ones dgemm): 2 M N nF flops (PBE: + 4 x 2 M n_s^2
+                 for SIC_ex), 8 M (N + nF) bytes
       vab        V^i_ab, symmetric pair blocks: sum_s M n_s^2 (n_s + 1) flops, 8 M 2 nF bytes
-    Peaks: FP64 MFMA 78.6 TFLOP/s for the dgemms, FP64 or FP32 MFMA for V^i_ab by form, HBM 8 TB/s."""
+    Peaks: FP64 MFMA 78.6 TFLOP/s for the products, FP64 or FP32 MFMA for V^i_ab by form, HBM 8 TB/s."""
     M, N, nF = float(counts[2]), float(counts[3]), float(counts[4])
     pbe = bool(sysm.xc)
     nd = 10.0 if pbe else 1.0
@@ -573,13 +581,7 @@ def main() -> int:
     flops = coulomb_flops(best["counts"])
     arith, peak = PEAK[best["prec"]]
     kname = coulomb_kernel_name(best["prec"])
-    # compulsory HBM bytes of one launch: H once in the form's operand layout, V written once, mesh coordinates
-    c = best["counts"]
-    hbytes = {"fp64": 8, "mixed": 4, "bf16x3": 6, "bf16x2": 4}[best["prec"]]
-    nfl = int(c[4])
-    cols = 64 if nfl <= 64 else 128 if nfl <= 128 else 192 if nfl <= 192 else 256
-    ldh = (nfl + cols - 1) // cols * cols
-    alg_bytes = float(c[6]) * ldh * hbytes + 8.0 * c[2] * c[4] + 24.0 * c[2]
+    alg_bytes = coulomb_bytes(best["counts"], best["prec"])
     achieved = flops / (best["kernel_ms"] * 1e-3) / 1e12
     counts = best["counts"]
     out = {
