@@ -200,22 +200,23 @@ int32_t flosic_get_timings(flosic_ctx *ctx, int32_t n, double *ms);
  * [2] nmsh [3] nbas [4] nflo (both spins) [5] exponent-pair groups [6] Hermite rows as the Coulomb kernel of
  * the current precision streams them (chunks zero-extended to its MFMA K step) [7] peak device bytes the
  * context has held since its creation [8] FLO columns per Coulomb block in use (0 for the VALU form) [9] (64-point
- * tile, Hermite row) pairs of the split-BF16 stream contracted with two pieces (far chunks, flosic_set_far_threshold;
+ * tile, Hermite row) pairs of the split-BF16 stream contracted with two pieces of H (far chunks, flosic_set_far_threshold;
  * 0 for the other forms).  n <= 10 values are written. */
 int32_t flosic_get_counts(flosic_ctx *ctx, int32_t n, int64_t *counts);
 
-/* Tile shape of the Coulomb kernels: FLO columns per block (each block contracts 64 mesh points with this many
- * columns; a narrower block repeats the Boys/Hermite R generation for every column block but gives more blocks).
+/* Tile shape of the Coulomb kernels: the most FLO columns per block (each block contracts 64 mesh points with at most this
+ * many columns and at most 192, the FLOs shared out evenly in tiles of 16; a narrower block repeats the Boys/Hermite R
+ * generation for every column block but gives more blocks).
  * 0 (default): the widest the precision allows; 64, 128, 192, 256: fixed (must divide the padded FLO count:
  * 64, 128, 192 or a multiple of 256; the split-BF16 forms take at most 192); -1: autotuned at the next
- * evaluation, every legal width timed on a strided sample of <= 32768 mesh points and the fastest kept (cached
- * per process by precision, FLO count, Hermite rows and mesh size).  No reference counterpart. */
+ * evaluation, every legal width that gives another launch timed on a strided sample of <= 32768 mesh points and the
+ * fastest kept (cached per process by precision, FLO count, Hermite rows and mesh size).  No reference counterpart. */
 int32_t flosic_set_coulomb_cols(flosic_ctx *ctx, int32_t ncols);
 
 /* Far chunks of the three-piece split-BF16 form (FLOSIC_PREC_BF16X3).  A (64-point tile, chunk of exponent-pair
  * groups) pair whose every (point, group) pair has T = p|r - P|^2 > tfar (p the summed exponent and P the centre of
  * the pair's Gaussian product, bounded from below through the tile's centroid and radius) is contracted with two
- * bf16 pieces of R and H (3 products) instead of three (6 products); every other pair keeps three.  tfar <= 0 turns
+ * bf16 pieces of H instead of three (R keeps three; the third of H counts as zero); every other pair keeps three.  tfar <= 0 turns
  * this off; the default is 30, POISSON1's THIRTYSOMETHING (poisson1.f:101), whose RCUT = sqrt(30/DELTA_MIN) + DMAX
  * (poisson1.f:528) is where the reference's default mode hands a pair batch to its multipole far field.  The bits
  * are built once per mesh, basis and threshold.  No reference counterpart. */

@@ -66,7 +66,7 @@ void host_parallel(int n, F &&f, bool worth = true) {
 
 constexpr int kNcart[3] = {1, 3, 6};
 constexpr double kZed = 1.0e-30;  // coupot_sic.F:61
-// three-piece split-BF16 Coulomb: (tile, chunk) pairs whose every T = p|r - P|^2 exceeds this run with two pieces.
+// three-piece split-BF16 Coulomb: (tile, chunk) pairs whose every T = p|r - P|^2 exceeds this run with two pieces of H.
 // 30 is POISSON1's THIRTYSOMETHING (poisson1.f:101): beyond RCUT = sqrt(30/DELTA_MIN) + DMAX (poisson1.f:528) the
 // reference replaces the exact pair integrals by its multipole far field.
 constexpr double kFarTDefault = 30.0;
@@ -1108,7 +1108,6 @@ CoulJob<T> coulomb_job(const flosic_ctx *c, int nfb) {
     J.ldv = c->M;
     J.nsteps = form == COUL_BF16 ? c->rows_padded_bf16 / 32 : c->rows_padded / 4;
     J.ncb = coulomb_col_blocks(c->nF, nfb);
-    J.nfb = nfb;
     const bool far = form == COUL_BF16 && c->prec == FLOSIC_PREC_BF16X3 && c->far_ok && c->far_words > 0;
     J.far = far ? c->d_far.p : nullptr;
     J.farw = far ? c->far_words : 0;
@@ -1328,9 +1327,6 @@ int eval_coulomb(flosic_ctx *c) {
     return 0;
 }
 
-// Phase C: FLOs on the mesh, XC, total potential, energies, SIC matrix and V^i_ab.  With resident planes the mesh
-// is one block; in mesh-block mode the planes, FLO fields, V_tot and U of each block are built, used and dropped,
-// and G, V^i_ab accumulate over the blocks in block order.
 // offsets (doubles) in d_res: energy sums (9 per FLO), V_H of every FLO at the outermost point, -SIC(j,i) (nwf x nocc) of both
 // spins, -SIC_ex (nocc x nocc, PBE) of both spins
 struct ResLayout {
@@ -1370,6 +1366,9 @@ void take_results(flosic_ctx *c) {
     }
 }
 
+// Phase C: FLOs on the mesh, XC, total potential, energies, SIC matrix and V^i_ab.  With resident planes the mesh
+// is one block; in mesh-block mode the planes, FLO fields, V_tot and U of each block are built, used and dropped,
+// and G, V^i_ab accumulate over the blocks in block order.
 // overlap_host: with the fields resident (no mesh blocks), queue the host's results before the V^i_ab kernels so that
 // the host works on them while those kernels run (single evaluations; a batch keeps its captured region free of
 // copies to host memory)

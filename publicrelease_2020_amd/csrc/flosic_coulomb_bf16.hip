@@ -32,8 +32,9 @@ namespace flosic {
 // 3.4e4 points) 0.279 -> 0.097 ms; 30 FLOs (1686, 1.2e5) 2.98 -> 1.18; 48 FLOs (4163, 1.9e5) 12.6 -> 5.1; 64 FLOs (7371,
 // 2.4e5) 25.8 -> 17.5; 96 FLOs (15750, 3.7e5) 96.0 -> 68.2; 120 FLOs (24241, 3.1e5) 104 -> 85.5; 192 FLOs (60795, 2.0e5)
 // 242 -> 192.  With CW = 1 making R bounds the loop (32 and 48 FLOs take nearly the same time per row and point).  With
-// CW = 4 the MFMAs are 57% busy: of the 192 ms the MFMAs alone need 111, with A from LDS 118, with the FP64 sums 130, with
-// H from L2 (three quarters of a gigabyte per tile, 96% hits) 168; the rest is what the producers take from the consumers.
+// CW = 4 the MFMAs are 57% busy there (52% by counters at 7.4e5 points, 5.7e5 rows): of the 192 ms the MFMAs alone need 111,
+// with A from LDS 118, with the FP64 sums 130, with H from L2 (three quarters of a gigabyte per tile, 96% hits) 168; the rest
+// is what the producers take from the consumers.  In far chunks the product with the third piece of H runs on zeros.
 // ---------------------------------------------------------------------------------------------------
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v2f __attribute__((ext_vector_type(2)));

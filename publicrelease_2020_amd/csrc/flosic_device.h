@@ -257,13 +257,13 @@ template <> struct MfmaTraits<float> {
 // Batched Coulomb: one launch over the (system, point tile, column block) items of every system of one form.
 // Block b runs item b with the single-system tile code; the host orders the systems (heaviest items first) so
 // that the dispatcher, which hands blocks to CUs in index order as CUs free up, balances them like a work queue.
-// One block fills a CU (16 waves at 128 VGPRs), so the grid is the queue and no block loops.
+// The grid is the queue, two blocks of four waves (split-BF16: one of eight) per CU at a time, and no block loops.
 // ---------------------------------------------------------------------------------------------------
 // Every job of a batch form in one launch.  The job records sit in device memory (a batch of 48 systems does not fit
 // the kernel argument space); each block copies its job through readfirstlane word by word, so every field is a
 // scalar (uniform) value in the tile code, as when it comes from the kernel arguments, and the tile's loop bounds
-// stay scalar branches.  Jobs of different column-block widths share the launch: the block switches on its job's
-// width, and the LDS of the widest tile is shared by all widths.
+// stay scalar branches.  Jobs of different splits share the launch: the block switches on the column waves
+// that its job's column tiles ask for, and all splits share the LDS of the largest.
 template <typename T>
 __device__ __forceinline__ CoulJob<T> uniform_job(const CoulJob<T> *__restrict__ jobs, int j) {
     static_assert(sizeof(CoulJob<T>) % 4 == 0, "job record in 32-bit words");

@@ -40,12 +40,13 @@ struct PairDev {
     double sym;          // 2 for cA != cB, else 1
 };
 
-// chunk of consecutive groups of one order L (split-BF16 forms): Hermite rows [hrow0, hrow0 + (pe-pb)*ntuv(L)) staged
-// in LDS and zero-extended to kr rows (a multiple of the MFMA K step)
+// chunk of consecutive groups of one order L (split-BF16 forms): Hermite rows [hrow0, hrow0 + (pe-pb)*ntuv(L)), zero-extended
+// to kr rows (a multiple of the MFMA K step); R of a chunk is made at a time
 constexpr int kChunkRowsBf16 = 64;  // split-BF16 kernel: K step 32
 constexpr int kFarWords = 1000;     // most 32-bit words of far-chunk bits per tile (32000 chunks)
 struct ChunkDev {
-    // groups [pb, pe); L: their Hermite order, or 5 / 6 for the first 32 / last 3 rows of L = 4 groups; kr: rows after zero extension; hrow0: first Hermite row of group pb
+    // groups [pb, pe); L: their Hermite order, or 5 / 6 for the first 32 / last 3 rows of L = 4 groups; kr: rows after zero
+    // extension; hrow0: first Hermite row of group pb
     int pb, pe, L, kr, hrow0;
     int prow0;  // first row of the chunk in the zero-extended row space of its list (split-BF16 H layout)
     int flush;  // the FP32 accumulators go into the FP64 sums after this chunk
@@ -63,7 +64,7 @@ struct FpSegs {
 
 // One system's Coulomb contraction as the kernels see it.  H is in the operand order of the form (double or
 // float fragments over K steps of 4 rows, or bf16 pieces over K steps of 32 rows: nsteps steps); ncb column
-// blocks (split-BF16: of nfb columns; FP forms: the nct column tiles shared out evenly); V[f * ldv + k].  The FP forms
+// blocks, the nct column tiles shared out evenly over them; V[f * ldv + k].  The FP forms
 // walk the groups by seg, the split-BF16 forms by the chunk list.
 template <typename T>
 struct CoulJob {
@@ -79,7 +80,6 @@ struct CoulJob {
     int64_t ldv;
     int64_t nsteps;
     int ncb;
-    int nfb;  // FLO columns per block (the single-launch batch kernels switch on it)
     // three-piece split-BF16 form: far-chunk bits of every 64-point tile (farw words per tile), or null
     const unsigned *far;
     int farw;
@@ -92,7 +92,7 @@ struct CoulJob {
 // split-BF16 form takes at most 192
 bool coulomb_cols_legal(int nfb, int ldh, bool split);
 
-// FLO columns handled by one Coulomb block: all of them up to 256
+// The default width: all FLOs up to 256 columns, of which a block takes at most 192 (coulomb_col_blocks)
 int coulomb_cols(int nF);
 
 // per-phase launch helpers (stream-ordered)
@@ -142,8 +142,9 @@ void launch_coulomb_mfma(const FpSegs &seg, const double4 *pairP, const T *Hf, c
                          int nfb = 0);
 
 // Batched form: every job of one Coulomb form in one launch over the (system, point tile, column block) items; the
-// job records and the item offsets in device memory (off[j] the first item of job j, which has ceil(M/64) * ncb items,
-// tile-major; off[njobs] the total, < 2^31), each job with its own column-block width (jobs[j].nfb).
+// job records and the item offsets in device memory (off[j] the first item of job j, which has ncb items for every
+// 64-point tile, in the split-BF16 form for every bf16_items work item, tile-major; off[njobs] the total, < 2^31), each job
+// with its own column blocks (jobs[j].nct, ncb).
 template <typename T>
 void launch_coulomb_batch_all(const CoulJob<T> *jobs, const int64_t *off, int njobs, int64_t items,
                               const double *btab, hipStream_t s);

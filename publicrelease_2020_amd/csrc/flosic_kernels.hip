@@ -359,8 +359,9 @@ void launch_coulomb(const int *segL, const double4 *pairP, const int *pairRow, c
                        pairRow, H, ldh, x, y, z, M, btab, nF, V, ldv);
 }
 
-// FLO columns per Coulomb block: all of them up to 256 (ldh is nF rounded up to a multiple of this); the
-// split-BF16 kernel takes at most 192 (its register budget), 128 beyond that
+// Column-block widths: by default all FLOs up to 256 columns (ldh is nF rounded up to a multiple of this), in the split-BF16
+// form up to 192 and 128 beyond that.  A block takes at most 12 tiles of 16 columns, four column waves of three, whatever
+// width is asked for (coulomb_col_blocks).
 int coulomb_cols(int nF) { return nF <= 64 ? 64 : nF <= 128 ? 128 : nF <= 192 ? 192 : 256; }
 bool coulomb_cols_legal(int nfb, int ldh, bool split) {
     if (nfb != 64 && nfb != 128 && nfb != 192 && nfb != 256) return false;

@@ -326,8 +326,8 @@ class Flosic:
         return c
 
     def set_far_threshold(self, tfar: float):
-        """Three-piece split-BF16 form: (tile, chunk) pairs with every T = p|r-P|^2 > tfar run with two pieces;
-        tfar <= 0 keeps three pieces everywhere."""
+        """Three-piece split-BF16 form: (tile, chunk) pairs with every T = p|r-P|^2 > tfar run with two pieces
+        of H; tfar <= 0 keeps three pieces everywhere."""
         self._chk(self._L.flosic_set_far_threshold(self._h, float(tfar)))
 
     def set_coulomb_cols(self, ncols: int):
