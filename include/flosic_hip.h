@@ -199,7 +199,7 @@ int32_t flosic_get_timings(flosic_ctx *ctx, int32_t n, double *ms);
  * rows (shell pairs that share both primitive exponents and centres are one group with one row block)
  * [2] nmsh [3] nbas [4] nflo (both spins) [5] exponent-pair groups [6] Hermite rows as the Coulomb kernel of
  * the current precision streams them (chunks zero-extended to its MFMA K step) [7] peak device bytes the
- * context has held since its creation [8] FLO columns per Coulomb block in use (0 for the VALU form) [9] (64-point
+ * context has held since its creation [8] column-block width in use (flosic_set_coulomb_cols; 0 for the VALU form) [9] (64-point
  * tile, Hermite row) pairs of the split-BF16 stream contracted with two pieces of H (far chunks, flosic_set_far_threshold;
  * 0 for the other forms).  n <= 10 values are written. */
 int32_t flosic_get_counts(flosic_ctx *ctx, int32_t n, int64_t *counts);

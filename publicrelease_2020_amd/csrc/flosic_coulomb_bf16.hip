@@ -648,7 +648,8 @@ __device__ __forceinline__ void bf_consumer(unsigned char *__restrict__ lds, BfT
 // Waves per tile with CW = 1.  Two tiles of four waves share the H that they read at the same time, one tile of eight leaves
 // less of the chip idle in the last round of 256 blocks: 48 FLOs, 2903 tiles 5.07 and 5.64 ms; 30 FLOs, 1816 tiles 1.18 and
 // 1.24; 10 FLOs, 530 tiles 0.125 and 0.097.  So eight where that saves more than a tenth of the rounds (a round of two tiles
-// counts twice).
+// counts twice).  In a batch the systems share a launch and only the last of them has such a round, yet the split is
+// each system's own, so that it has the bits of its single launch.
 __host__ __device__ inline int bf_runs(int64_t M) {
     const int64_t tiles = (M + 63) / 64;
     return 11 * ((tiles + 255) / 256) < 20 * ((tiles + 511) / 512) ? 8 : 4;
